@@ -28,7 +28,8 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libnesle_hip.so"
-HIP_SOURCES = [CSRC / "nes_step.hip", CSRC / "nes_step_full.hip", CSRC / "nes_step_narrow.hip", CSRC / "nes_kernels.hip",
+HIP_SOURCES = [CSRC / "nes_step.hip", CSRC / "nes_step_full.hip", CSRC / "nes_step_narrow.hip", CSRC / "nes_step_wave.hip", CSRC / "nes_step_solo.hip",
+               CSRC / "nes_kernels.hip",
                CSRC / "nes_render.hip", CSRC / "nes_host.hip", CSRC / "ppo_head.hip", CSRC / "smb_shaped.hip"]
 SHIM_SOURCE = CSRC / "cuda_core_module.cpp"
 

@@ -139,6 +139,10 @@ struct DeviceState {
     std::uint8_t* lat_sx;      // [n]
     std::uint8_t* lat_sy;      // [n]
     std::uint8_t* lat_ctrl;    // [n]
+
+    // No instruction that program flow can fall into among the vectors
+    // reaches past the PRG image (nes_step_wave.hip runs the batch then).
+    std::uint32_t closed_end;
 };
 
 // Step-kernel census (stats mode 3): what the waves of one launch did, summed

@@ -60,6 +60,11 @@
 #include "nes_layout.h"
 #include "nes_micro.h"
 
+// Which of the step kernel's translation units this is (see launch_step).
+#ifndef NESLE_STEP_PART
+#define NESLE_STEP_PART 0
+#endif
+
 namespace nesle {
 namespace {
 
@@ -68,7 +73,14 @@ __constant__ mc::Table c_micro_full = mc::kTableFull;
 
 // The whole 160 KB of a CU's LDS, statically: one workgroup per CU, and a
 // static array has a known address (0), so LDS addresses need no base add.
+#if NESLE_STEP_PART == 3
+// One console per wave (nes_step_wave.hip): two workgroups of 16 waves per CU.
+constexpr std::uint32_t kLdsLimit = 67584;
+constexpr std::uint32_t kLdsRom = 256;
+#else
 constexpr std::uint32_t kLdsLimit = 160u * 1024u;
+constexpr std::uint32_t kLdsRom = 0;            // the PRG image
+#endif
 __shared__ __attribute__((aligned(16))) std::uint8_t lds[kLdsLimit];
 
 constexpr std::uint32_t kMaxBlock = 1024;       // up to 16 waves per workgroup
@@ -223,21 +235,27 @@ struct Console {
     __device__ __forceinline__ void set_oam_data(std::uint32_t v) { flags = (flags & ~0xFF0000u) | ((v & 0xFF) << 16); }
 
     // ---- LDS register area ----------------------------------------------------------
-    __device__ __forceinline__ std::uint32_t r8(std::uint32_t f) const { return lds[base + kRegs + f]; }
+#if NESLE_STEP_PART == 3
+    std::uint32_t regs_base = 0;   // the wave kernel keeps the area apart from the RAM
+    __device__ __forceinline__ std::uint32_t regs_at() const { return regs_base; }
+#else
+    __device__ __forceinline__ std::uint32_t regs_at() const { return base + kRegs; }
+#endif
+    __device__ __forceinline__ std::uint32_t r8(std::uint32_t f) const { return lds[regs_at() + f]; }
     __device__ __forceinline__ void w8(std::uint32_t f, std::uint32_t v) const {
-        lds[base + kRegs + f] = static_cast<std::uint8_t>(v);
+        lds[regs_at() + f] = static_cast<std::uint8_t>(v);
     }
     __device__ __forceinline__ std::uint32_t r16(std::uint32_t f) const {
-        return *reinterpret_cast<const std::uint16_t*>(lds + base + kRegs + f);
+        return *reinterpret_cast<const std::uint16_t*>(lds + regs_at() + f);
     }
     __device__ __forceinline__ void w16(std::uint32_t f, std::uint32_t v) const {
-        *reinterpret_cast<std::uint16_t*>(lds + base + kRegs + f) = static_cast<std::uint16_t>(v);
+        *reinterpret_cast<std::uint16_t*>(lds + regs_at() + f) = static_cast<std::uint16_t>(v);
     }
     __device__ __forceinline__ std::uint32_t r32(std::uint32_t f) const {
-        return *reinterpret_cast<const std::uint32_t*>(lds + base + kRegs + f);
+        return *reinterpret_cast<const std::uint32_t*>(lds + regs_at() + f);
     }
     __device__ __forceinline__ void w32(std::uint32_t f, std::uint32_t v) const {
-        *reinterpret_cast<std::uint32_t*>(lds + base + kRegs + f) = v;
+        *reinterpret_cast<std::uint32_t*>(lds + regs_at() + f) = v;
     }
 
     // ---- console RAM ($0000-$07FF, mirrored to $1FFF) -------------------------
@@ -462,7 +480,7 @@ struct Console {
     // ---- CPU bus (console.hpp:49-101) --------------------------------------------
     __device__ std::uint32_t bus_rd(std::uint32_t addr) {
         if (addr < 0x2000) return ram_rd(addr & 0x7FF);
-        if (addr >= 0x8000) return lds[addr & 0x7FFF];
+        if (addr >= 0x8000) return lds[kLdsRom + (addr & 0x7FFF)];
         if (addr >= 0x6000) return s->ram[goff(addr - 0x5800)];
         return io_rd(addr) & 0xFF;
     }
@@ -1393,19 +1411,18 @@ __global__ void __launch_bounds__(kFull ? 256 : kMaxBlock) step_kernel(DeviceSta
     }
 }
 
-// Which of the step kernel's translation units this is (see launch_step).
-#ifndef NESLE_STEP_PART
-#define NESLE_STEP_PART 0
-#endif
 // Split-layout launches with at most 2^5 consoles per wave take the
 // nes_step_narrow.hip instances.
 constexpr std::uint32_t kNarrowLaneBits = 5;
+// One console per wave (launch_step).
+[[maybe_unused]] constexpr std::uint32_t kSoloMaxConsoles = 4096, kWaveMaxConsoles = 32768;
 
 struct Geometry {
     std::uint32_t waves, lane_bits, consoles, blocks, lds;
     bool full;
 };
 
+#if NESLE_STEP_PART != 3
 // W waves per workgroup (one workgroup per CU), L consoles per wave: the
 // smallest power-of-two L with 256 CUs x W x L >= n.  W trades issue slots for
 // latency hiding: W/4 waves share each SIMD.
@@ -1434,12 +1451,14 @@ hipError_t launch_variant(const DeviceState& s, const Geometry& g, std::uint32_t
     return hipGetLastError();
 }
 
+// A frame needs at most ceil(89,342 / 6) = 14,891 instructions.
+bool budget_binds(std::uint32_t max_instr) { return max_instr < 15000; }
+
 // One layout's kernels, for every statistics mode and frame budget.
 template <bool kFull>
 hipError_t launch_layout(const DeviceState& s, const Geometry& g, std::uint32_t frameskip, std::uint32_t max_instr,
                          int stats_mode, hipStream_t stream) {
-    // A frame needs at most ceil(89,342 / 6) = 14,891 instructions.
-    const bool budget = max_instr < 15000;
+    const bool budget = budget_binds(max_instr);
     if (stats_mode == 3) return launch_variant<3, kFull, true>(s, g, frameskip, max_instr, stream);
     if (stats_mode == 2) return launch_variant<2, kFull, true>(s, g, frameskip, max_instr, stream);
     if (stats_mode == 1) return launch_variant<1, kFull, true>(s, g, frameskip, max_instr, stream);
@@ -1447,6 +1466,7 @@ hipError_t launch_layout(const DeviceState& s, const Geometry& g, std::uint32_t 
                   : launch_variant<0, kFull, false>(s, g, frameskip, max_instr, stream);
 }
 
+#endif
 #if NESLE_STEP_PART == 0
 // Waves per workgroup: NESLE_WAVES_PER_GROUP (4, 8 or 16) overrides the default.
 std::uint32_t waves_per_group() {
@@ -1466,12 +1486,17 @@ std::uint32_t waves_per_group() {
 // (NESLE_STEP_PART 0: the split layout at 64 consoles per wave, and
 // launch_step), nes_step_full.hip (1: all RAM in LDS) and
 // nes_step_narrow.hip (2: the split layout at 16 or 32 consoles per wave).
+// nes_step_wave.hip and nes_step_solo.hip (3) hold another kernel, one
+// console per wave, around this file's console routines; launch_step gives
+// it the batches it is quicker on.
 // Each part recomputes the geometry from the console count and waves per
 // workgroup, as launch_step does.
 hipError_t launch_step_full(const DeviceState& s, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
                             hipStream_t stream);
 hipError_t launch_step_narrow(const DeviceState& s, std::uint32_t waves, std::uint32_t frameskip,
                               std::uint32_t max_instr, int stats_mode, hipStream_t stream);
+hipError_t launch_step_wave(const DeviceState& s, std::uint32_t frameskip, hipStream_t stream);
+hipError_t launch_step_solo(const DeviceState& s, std::uint32_t frameskip, hipStream_t stream);
 
 #if NESLE_STEP_PART == 1
 hipError_t launch_step_full(const DeviceState& s, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
@@ -1487,9 +1512,17 @@ hipError_t launch_step_narrow(const DeviceState& s, std::uint32_t waves, std::ui
     if (g.full || g.lane_bits > kNarrowLaneBits || g.lds > kLdsLimit) return hipErrorInvalidConfiguration;
     return launch_layout<false>(s, g, frameskip, max_instr, stats_mode, stream);
 }
-#else
+#elif NESLE_STEP_PART == 0
 hipError_t launch_step(const DeviceState& s, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
                        hipStream_t stream) {
+    // One console per wave up to 32,768 consoles: there the wave kernel takes
+    // 13.2 ms on a program that never idles and 4.75 on one that waits in
+    // JMP *, this file's 17.3 and 5.98; at 40,960 16.7 and about 6 against
+    // 18.6 and 6.03.  Its solo form up to 4,096, four waves per SIMD: 2.74 ms
+    // there against 2.81, 2.46 against 2.80 at 1,000; at 8,192 3.92 against
+    // 3.43.
+    if (stats_mode == 0 && !budget_binds(max_instr) && s.closed_end != 0 && s.n <= kWaveMaxConsoles)
+        return s.n <= kSoloMaxConsoles ? launch_step_solo(s, frameskip, stream) : launch_step_wave(s, frameskip, stream);
     const std::uint32_t waves = waves_per_group();
     const Geometry g = geometry(s.n, waves);
     if (g.full) return launch_step_full(s, frameskip, max_instr, stats_mode, stream);

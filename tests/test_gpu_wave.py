@@ -1,0 +1,135 @@
+"""The one-console-per-wave step kernels (nes_step_wave.hip, nes_step_solo.hip),
+which run plain steps of up to 32,768 consoles.  A statistics step runs the
+lane kernel, which the oracle tests pin, so twin batches stepped with and
+without statistics must agree in every byte: over programs that take each
+side path (I/O, PRG RAM, code in RAM, stack and address wraps, illegal
+opcodes, OAM DMA from every kind of page, the idle loop) and over sizes at the
+edges of the workgroup shapes.  Programs that run into and over the vectors
+are compared with the oracle itself."""
+
+from __future__ import annotations
+
+import re
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from nesle_amd import abi, build, synthrom
+from oracle import oracle as O
+from tests.helpers import first_diff, masks_for, say
+from tests.kat_roms import nrom_bytes
+from tests.test_gpu_features import address_wrap_rom, feature_rom, io_corner_rom, oam_rom, stack_wrap_rom
+from tests.test_gpu_idle import idle_rom
+
+ROMS = {
+    "random": lambda: synthrom.make_rom(5).rom,
+    "nrom128": lambda: synthrom.make_rom(6, prg_banks=1).rom,
+    "split": lambda: synthrom.make_rom(7, split=True).rom,
+    "idle": idle_rom,
+    "features": feature_rom,
+    "oam": oam_rom,
+    "stack_wrap": stack_wrap_rom,
+    "io_corner": io_corner_rom,
+    "address_wrap": address_wrap_rom,
+}
+
+
+def twins(rom: bytes, n: int, frameskip: int, steps: int, seed: int) -> None:
+    a, b = abi.Batch(rom, n, frameskip=frameskip), abi.Batch(rom, n, frameskip=frameskip)
+    sample = sorted({0, 1 % n, n // 2, n - 1, *np.random.default_rng(n).integers(0, n, 12).tolist()})
+    for k in range(steps):
+        m = masks_for(seed, n, k)
+        for batch, stats in ((a, 0), (b, 1)):
+            batch.set_actions(m)
+            batch.step(auto_reset=k % 3 == 1, stats_mode=stats)
+        for view in (abi.VIEW_REWARDS, abi.VIEW_DONES, abi.VIEW_RAM):
+            assert np.array_equal(a.host(view), b.host(view)), f"step {k} view {view}"
+    # A console stopped by an illegal opcode in the middle of a step keeps the
+    # step's earlier vblank only under statistics (which capture every one).
+    for e in np.flatnonzero((a.host(abi.VIEW_PRESENT) != b.host(abi.VIEW_PRESENT)).any(axis=1)):
+        assert a.save_state(int(e))[O.OFF["fault"]] & 1, f"presentation record of console {e}"
+    for e in sample:
+        got, want = a.save_state(e), b.save_state(e)
+        assert np.array_equal(got, want), f"console {e}: {first_diff(got, want)}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(ROMS))
+@pytest.mark.parametrize("n", [60, 4160])
+def test_programs_agree_with_the_lane_kernel(name, n):
+    """60 consoles: the solo form; 4,160: two workgroups on some CUs."""
+    say(f"[gpu] wave kernel: {name} N={n}")
+    twins(ROMS[name](), n, 4, 9, 31)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,frameskip", [(1, 1), (2, 3), (257, 4), (700, 2), (1500, 4), (2814, 4), (4096, 1), (4097, 5),
+                                         (8200, 4), (32768, 1)])
+def test_sizes_agree_with_the_lane_kernel(n, frameskip):
+    """1, 2, 4, 8, 12 and 16 waves per workgroup, the last one ragged (2,814
+    consoles in workgroups of 12 end past the row pitch of 2,816), the ends of
+    both forms' ranges."""
+    say(f"[gpu] wave kernel: N={n} fs={frameskip}")
+    twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 77)
+
+
+def vector_rom(irq: int, flow: list[int]) -> bytes:
+    """Flow at $FFF5 (padded with NOPs) into vectors whose bytes are all NOPs
+    but the last; the code they point to counts and comes back."""
+    back = [0xE6, 0x20, 0xA5, 0x20, 0x85, 0x00, 0x49, 0xFF, 0x85, 0x01, 0x4C, 0xF5, 0xFF]   # count; JMP $FFF5
+    return nrom_bytes(2, code={0xEAEA: back, irq: back, 0xFFF5: (flow + [0xEA] * 5)[:5]}, reset=0xEAEA, nmi=0xEAEA, irq=irq)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("irq,flow", [
+    (0xEAEA, []),                    # NOPs over the end: the next instruction is RAM's
+    (0xADEA, []),                    # LDA abs at $FFFF: its operand is RAM $0000-$0001
+    (0xA5EA, []),                    # LDA zp at $FFFF
+    (0xEA8D, []),                    # STA abs at $FFFE
+    (0xADEA, [0x4C, 0xFF, 0xFF]),    # the same instruction entered by a jump
+    (0xEAEA, [0x18, 0x90, 0x06]),    # a branch over the end
+    (0x9090, [0x18, 0x90, 0x02]),    # a branch to the vectors
+])
+def test_flow_over_the_vectors_matches_oracle(irq, flow):
+    rom = vector_rom(irq, flow)
+    b, cons = abi.Batch(rom, 3, frameskip=2), [O.Oracle(rom) for _ in range(3)]
+    for c in cons:
+        c.set_reward()
+    stopped = set()
+    for k in range(4):
+        m = masks_for(3, 3, k)
+        b.set_actions(m)
+        b.step()
+        for e, c in enumerate(cons):
+            if e in stopped:
+                continue
+            try:
+                c.step(int(m[e]), 2)
+            except RuntimeError:       # an illegal opcode: the oracle's PC has moved past it
+                stopped.add(e)
+                assert b.save_state(e)[O.OFF["fault"]] & 1
+                continue
+            got, want = b.save_state(e), c.save()
+            assert np.array_equal(got, want), f"step {k} console {e}: {first_diff(got, want)}"
+
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not available")
+@pytest.mark.parametrize("source", ["nes_step_wave.hip", "nes_step_solo.hip"])
+def test_two_workgroups_share_a_cu(tmp_path, source):
+    """Eight waves per SIMD: at most 80 KB of LDS, 80 scalar registers (800
+    per SIMD in units of 16) and 64 vector registers, and no scratch."""
+    out = tmp_path / "wave.s"
+    path = build.CSRC / source
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-device-only", "-S", *build.source_flags(path), "-o",
+                    str(out), str(path)], check=True, capture_output=True, text=True)
+    meta = out.read_text().split("amdhsa.kernels:", 1)[1]
+    value = {k: int(v) for k, v in re.findall(r"\.(group_segment_fixed_size|private_segment_fixed_size|sgpr_count|"
+                                              r"vgpr_count):\s+(\d+)", meta)}
+    assert value["group_segment_fixed_size"] <= 80 * 1024 and value["private_segment_fixed_size"] == 0
+    assert value["sgpr_count"] <= 80 and value["vgpr_count"] <= 64
