@@ -140,10 +140,13 @@ struct DeviceState {
     std::uint8_t* lat_sy;      // [n]
     std::uint8_t* lat_ctrl;    // [n]
 
-    // No instruction that program flow can fall into among the vectors
-    // reaches past the PRG image (nes_step_wave.hip runs the batch then).
-    std::uint32_t closed_end;
+    // The one-console-per-wave kernels may run this step (nes_host.hip says
+    // when), and where they report how often their general path was taken:
+    // kGeneralSlots words of host memory.
+    std::uint32_t per_wave;
+    std::uint32_t* general;
 };
+constexpr std::uint32_t kGeneralSlots = 16;
 
 // Step-kernel census (stats mode 3): what the waves of one launch did, summed
 // over waves.  A "wave-iteration" is one trip of the step loop (one emulated

@@ -1521,7 +1521,7 @@ hipError_t launch_step(const DeviceState& s, std::uint32_t frameskip, std::uint3
     // 18.6 and 6.03.  Its solo form up to 4,096, four waves per SIMD: 2.74 ms
     // there against 2.81, 2.46 against 2.80 at 1,000; at 8,192 3.92 against
     // 3.43.
-    if (stats_mode == 0 && !budget_binds(max_instr) && s.closed_end != 0 && s.n <= kWaveMaxConsoles)
+    if (stats_mode == 0 && !budget_binds(max_instr) && s.per_wave != 0 && s.n <= kWaveMaxConsoles)
         return s.n <= kSoloMaxConsoles ? launch_step_solo(s, frameskip, stream) : launch_step_wave(s, frameskip, stream);
     const std::uint32_t waves = waves_per_group();
     const Geometry g = geometry(s.n, waves);

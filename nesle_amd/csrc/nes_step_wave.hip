@@ -23,7 +23,10 @@
 // 8,192 consoles 6.9 ms instead of 5.1 when it was so).
 //
 // Statistics and binding instruction budgets stay with the lane kernel, as do
-// images whose flow can run past their end (DeviceState::closed_end).
+// images whose flow can run past their end, and programs that take the general
+// path too often (nes_host.hip): an instruction there costs about 1,100
+// cycles of a SIMD, where a lane of the lane kernel shares 1,400 with 63
+// others.
 //
 // Built twice: this file's own instance for many waves per SIMD, and
 // nes_step_solo.hip's for few (SOLO in nes_wave.h).
@@ -154,6 +157,7 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
         cpu.sp = uni(s.sp[env]); cpu.p = uni(s.p[env]);
         cpu.left = static_cast<std::int32_t>(uni(horizon0));
         __builtin_amdgcn_s_setprio(3);
+        std::uint32_t general = 0;   // trips through the general path
         bool active = !(c.flags & kFault) && frameskip != 0;
         while (active) {
             const bool nmi = (c.flags & kNmiPending) != 0;
@@ -168,6 +172,7 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
                 c.flags = cpu.flags;
             }
             c.s = reload(c.s);
+            general += why != kWaveEvent ? 1u : 0u;
             if (why == kWaveStore) {
                 const std::uint32_t at = cpu.addr & 0xFFFF;
                 if (at < 0x2000) {
@@ -336,6 +341,9 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
         }
         flags = c.flags;
         frames = c.r32(reg::kFrames);
+        // How often the first consoles took the general path, per frame.
+        if (blockIdx.x < kGeneralSlots && wave == 0 && lane == 0 && frameskip != 0)
+            reload(c.s)->general[blockIdx.x] = general / frameskip;
     }
     __syncthreads();
 

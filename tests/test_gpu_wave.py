@@ -76,6 +76,38 @@ def test_sizes_agree_with_the_lane_kernel(n, frameskip):
     twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 77)
 
 
+def poll_rom() -> bytes:
+    """Reads of $2007 and $4015 and PRG RAM traffic without end: nearly every
+    instruction takes the general path."""
+    loop = [0xAD, 0x07, 0x20, 0x8D, 0x00, 0x60, 0xEE, 0x00, 0x60, 0xAD, 0x15, 0x40, 0x4C, 0x00, 0x80]
+    return nrom_bytes(2, code={0x8000: loop, 0x9000: [0x40]}, reset=0x8000, nmi=0x9000, irq=0x9000)
+
+
+@pytest.mark.gpu
+def test_polling_program_moves_to_the_lane_kernel():
+    """After its first steps the batch takes the lane kernel (quicker there);
+    the results stay the oracle's through the change and the trial steps."""
+    n, steps = 8200, 70
+    rom = poll_rom()
+    b, cons = abi.Batch(rom, n, frameskip=1), {e: O.Oracle(rom) for e in (0, 4100, n - 1)}
+    for c in cons.values():
+        c.set_reward()
+    b.set_timing(True)
+    took = []
+    for k in range(steps):
+        m = masks_for(8, n, k)
+        b.set_actions(m)
+        b.step()
+        before = sum(took)
+        took.append(b.timing()[0] - before)     # synchronises: the report is in
+        for e, c in cons.items():
+            c.step(int(m[e]), 1)
+    for e, c in cons.items():
+        got, want = b.save_state(e), c.save()
+        assert np.array_equal(got, want), f"console {e}: {first_diff(got, want)}"
+    assert max(took[2:60]) < 0.5 * took[0], took
+
+
 def vector_rom(irq: int, flow: list[int]) -> bytes:
     """Flow at $FFF5 (padded with NOPs) into vectors whose bytes are all NOPs
     but the last; the code they point to counts and comes back."""
