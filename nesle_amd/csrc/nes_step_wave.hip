@@ -71,6 +71,31 @@ __device__ __forceinline__ void yield(std::uint32_t frames_left, std::uint32_t d
     }
 }
 
+// A loop that waits for a PPUSTATUS flag: LDA or BIT $2002 at `pc`, which has
+// just read `v`, an AND # or none, and a branch back.  The flags change only
+// at PPU events and with the read itself (it clears bit 7, and the open bus
+// then holds what it read), so once bit 7 is clear every pass leaves the
+// registers as the one before, and the passes that end before the next event,
+// `left` dots away, are skipped: their dots are returned.
+__device__ __forceinline__ std::uint32_t waited(std::uint32_t pc, std::uint32_t v, std::uint32_t p, std::int32_t left) {
+    if (v & 0x80) return 0;
+    const std::uint8_t* at = lds + kLdsRom + (pc & 0x7FFF) + 3;
+    const std::uint32_t b0 = uni(at[0]), b1 = uni(at[1]), b2 = uni(at[2]), b3 = uni(at[3]);
+    const bool masked = b0 == 0x29;
+    const std::uint32_t op = masked ? b2 : b0, rel = masked ? b3 : b1, len = masked ? 7u : 5u;
+    if ((op & 0x1F) != 0x10 || rel != 0x100 - len) return 0;
+    if (masked) {   // the flags the AND leaves, of A (BIT does not load it: such a loop is not skipped)
+        if (uni(at[-3]) != 0xAD) return 0;
+        const std::uint32_t r = v & b1;
+        p = (p & ~0x82u) | (r & 0x80) | (r == 0 ? 2u : 0u);
+    }
+    const std::uint32_t* d = c_micro_full.e[op].d;
+    if (ubfe(p ^ ((d[2] >> 8) & 0xFF), d[2], d[3]) == 0) return 0;   // falls through
+    const std::uint32_t cross = (((pc + len) ^ pc) & 0xFF00) ? 1u : 0u;
+    const std::uint32_t pass = 3 * (4 + (masked ? 2 : 0) + 3 + cross);
+    return (static_cast<std::uint32_t>(left) - 1) / pass * pass;
+}
+
 __global__ void __launch_bounds__(64 * kWaveMaxWaves) __attribute__((amdgpu_num_sgpr(80)))
 NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
     using C = Console<true>;
@@ -272,6 +297,8 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
                     active = false;
                 }
                 cpu.left = static_cast<std::int32_t>(uni(static_cast<std::uint32_t>(cpu.left) - dots));
+                if ((mi == 0xAD || mi == 0x2C) && ea == 0x2002 && cpu.left > 0 && pc0 - 0x8000u < kWaveRomEnd - 8u)
+                    cpu.left -= static_cast<std::int32_t>(waited(pc0, M, cpu.p, cpu.left));
             }
             if (counted && cpu.left <= 0) {   // a timing event was crossed: settle the PPU
                 const std::uint32_t fc = c.settle(c.r32(reg::kHorizon) - static_cast<std::uint32_t>(cpu.left), false);

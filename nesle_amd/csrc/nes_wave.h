@@ -18,8 +18,10 @@
 //                 included (which may have reached the event);
 //   kWaveGeneral  the next instruction is for the general path (other I/O
 //                 reads, PRG RAM, illegal opcodes, JMP indirect, stack and
-//                 zero-page pointer wraps, a jump to itself, a target outside
-//                 PRG ROM or among the vectors): nothing of it has run.
+//                 zero-page pointer wraps, loops that wait -- a jump to
+//                 itself, a branch back to its read of $2002 --, a target
+//                 outside PRG ROM or among the vectors): nothing of it has
+//                 run.
 //
 // Registers.  The countdown holds the dots to the next event less one, so
 // that subtracting an instruction's dots borrows exactly when it reaches the
@@ -1127,6 +1129,12 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 ; PPUSTATUS: flags over the open bus's low bits; clears vblank, the pending
 ; NMI and the write toggle (io bits 0-7 open bus, 8-15 status).
 .Lw%=_ppustatus:
+  s_bfe_u32 s[rU], s[rW], 0x80008
+  s_cmp_eq_u32 s[rU], 0xAD
+  s_cbranch_scc1 .Lw%=_poll
+  s_cmp_eq_u32 s[rU], 0x2C
+  s_cbranch_scc1 .Lw%=_poll
+.Lw%=_status:
   s_lshr_b32 s[rM], s[rIO], 8
   s_and_b32 s[rM], s[rM], 0xE0
   s_and_b32 s[rT], s[rIO], 0x1F
@@ -1135,6 +1143,32 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_or_b32 s[rIO], s[rIO], s[rM]
   s_andn2_b32 s[rFL], s[rFL], 0x12
   s_setpc_b64 s[rCall:rCall+1]
+; LDA or BIT $2002 of a loop that waits for a flag (a branch back to it next,
+; or an AND between them): the general path skips to the next event.
+.Lw%=_poll:
+  s_waitcnt lgkmcnt(0)
+  v_readfirstlane_b32 s[rR], v[vW]
+  v_readfirstlane_b32 s[rU], v[vW+1]
+  s_lshr_b32 s[rR], s[rR], 24
+  s_cmp_eq_u32 s[rR], 0x29
+  s_cbranch_scc1 .Lw%=_poll3
+  s_and_b32 s[rR], s[rR], 0x1F
+  s_cmp_lg_u32 s[rR], 0x10
+  s_cbranch_scc1 .Lw%=_status
+  s_and_b32 s[rR], s[rU], s[rFF]
+  s_cmp_eq_u32 s[rR], 0xFB
+  s_cbranch_scc1 .Lw%=_general
+  s_branch .Lw%=_status
+.Lw%=_poll3:
+  s_bitcmp0_b32 s[rW], 15             ; LDA
+  s_cbranch_scc1 .Lw%=_status
+  s_bfe_u32 s[rR], s[rU], 0x50008
+  s_cmp_lg_u32 s[rR], 0x10
+  s_cbranch_scc1 .Lw%=_status
+  s_bfe_u32 s[rR], s[rU], 0x80010
+  s_cmp_eq_u32 s[rR], 0xF9
+  s_cbranch_scc1 .Lw%=_general
+  s_branch .Lw%=_status
 ; OAMDATA: the byte at OAMADDR, kept in flags bits 16-23.
 .Lw%=_oamdata:
   s_bfe_u32 s[rM], s[rFL], 0x80010

@@ -24,7 +24,32 @@ from tests.kat_roms import nrom_bytes
 from tests.test_gpu_features import address_wrap_rom, feature_rom, io_corner_rom, oam_rom, stack_wrap_rom
 from tests.test_gpu_idle import idle_rom
 
+def wait_rom() -> bytes:
+    """Loops that wait for PPUSTATUS flags, in every form the kernel skips and
+    some it must not: LDA or BIT, with and without AND #, across a page, with
+    the read's open-bus bits in play, a loop that falls through at once, one
+    whose branch leads elsewhere."""
+    def at(addr, *code):
+        return addr, list(code)
+
+    parts = dict([
+        at(0x8000, 0x78, 0xA2, 0xFF, 0x9A, 0xA9, 0x80, 0x8D, 0x00, 0x20, 0xA9, 0x18, 0x8D, 0x01, 0x20, 0x4C, 0x00, 0x81),
+        at(0x8100, 0xAD, 0x02, 0x20, 0x10, 0xFB, 0xE6, 0x20, 0x4C, 0xFC, 0x82),              # LDA; BPL (vblank)
+        at(0x82FC, 0x2C, 0x02, 0x20, 0x70, 0xFB, 0xE6, 0x21, 0x4C, 0xFB, 0x83),              # BIT; BVS, over a page
+        at(0x83FB, 0x2C, 0x02, 0x20, 0x50, 0xFB, 0xE6, 0x22, 0x4C, 0x00, 0x85),              # BIT; BVC, over a page
+        at(0x8500, 0xAD, 0x02, 0x20, 0x29, 0x40, 0xD0, 0xF9, 0xE6, 0x23, 0x4C, 0xF9, 0x86),  # LDA; AND #$40; BNE
+        at(0x86F9, 0xAD, 0x02, 0x20, 0x29, 0x40, 0xF0, 0xF9, 0xE6, 0x24, 0x85, 0x25),        # ... BEQ, over a page
+        at(0x8704, 0x8E, 0x05, 0x20, 0xAD, 0x02, 0x20, 0x29, 0x1F, 0x85, 0x26, 0xCA),        # open bus = X
+        at(0x870F, 0xAD, 0x02, 0x20, 0x30, 0xFB, 0x2C, 0x02, 0x20, 0x90, 0x02, 0xE6, 0x27),  # BMI; BCC elsewhere
+        at(0x871B, 0x2C, 0x02, 0x20, 0x29, 0xFF, 0xD0, 0xF9, 0x4C, 0x00, 0x81),              # BIT; AND #; BNE
+        at(0x9000, 0x48, 0xE6, 0x10, 0xA5, 0x10, 0x29, 0x03, 0xD0, 0x05, 0xA9, 0x00, 0x8D, 0x01, 0x20,
+           0xA9, 0x18, 0x8D, 0x01, 0x20, 0xAD, 0x16, 0x40, 0x85, 0x11, 0x68, 0x40),
+    ])
+    return nrom_bytes(2, code=parts, reset=0x8000, nmi=0x9000, irq=0x9000)
+
+
 ROMS = {
+    "wait": wait_rom,
     "random": lambda: synthrom.make_rom(5).rom,
     "nrom128": lambda: synthrom.make_rom(6, prg_banks=1).rom,
     "split": lambda: synthrom.make_rom(7, split=True).rom,
