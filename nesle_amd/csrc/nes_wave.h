@@ -10,8 +10,8 @@
 // `asm goto` an exit chain through all its labels), hence assembly.  The
 // block runs instructions from PRG ROM whose operands lie in RAM, PRG ROM, the
 // I/O registers programs poll ($2002, $2004, $4016) or those they write in
-// numbers (nametables through $2007, $2005, $2006, $4000-$4015 but $4014),
-// and leaves with
+// numbers ($2000, $2001, $2005, $2006, $2007 to the nametables, $4000-$4016
+// but $4014), and leaves with
 //   kWaveEvent    an instruction reached the next PPU event; it is complete;
 //   kWaveStore    the instruction stores `value` at `addr`, another register
 //                 or PRG RAM: all of it but the store is done, its time
@@ -158,30 +158,36 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 ; ---- fetch, time and dispatch ------------------------------------------------
 ; The next instruction's bytes are in the window already read, \len bytes on;
 ; the window of eight bytes at the next instruction is read for the one after
-; it.  \k LDS operations have been issued since the handler began.
+; it.  \k LDS operations have been issued since the handler began.  W is the
+; next instruction's from here on.
 .macro AHEAD len, k=0
   s_waitcnt lgkmcnt(\k)
   v_perm_b32 v[vT], v[vW+1], v[vW], s[rSel\len]
   v_add_u32 v[vF], \len, v[vF]
   ds_read_b64 v[vW:vW+1], v[vF]
-.endm
-.macro GO
   v_readfirstlane_b32 s[rW], v[vT]
+.endm
+; AIM forms the jump's target, GO jumps.
+.macro AIM
 .if SOLO
   s_pack_lh_b32_b16 s[rJ], s[rW], s[rQ]
 .else
   s_pack_lh_b32_b16 s[rJ], s[rW], s[rTab]
 .endif
+.endm
+.macro GO
   s_setpc_b64 s[rJ:rJ+1]
 .endm
-; A jump's instruction: its window at vF.
-.macro ENTER
-  ds_read_b64 v[vW:vW+1], v[vF]
+; After a jump: its window has been read at \at.
+.macro ENTER at, off=0
+  ds_read_b64 v[vW:vW+1], v[\at] offset:\off
 .endm
 .macro ENTERED
   s_waitcnt lgkmcnt(0)
   v_perm_b32 v[vT], v[vW+1], v[vW], s[rSel0]
   s_nop 0
+  v_readfirstlane_b32 s[rW], v[vT]
+  AIM
   GO
 .endm
 .macro TIME dots
@@ -202,6 +208,7 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 .endm
 .macro NEXT dots
   PASS \dots, .Lw%=_exit
+  AIM
   GO
 .endm
 ; Finishes an instruction that leaves the block in the middle of its read.
@@ -469,6 +476,7 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   AHEAD \len, 1
 .Lw%=_time\n:
   PASS \dots, .Lw%=_event\n
+  AIM
   s_waitcnt lgkmcnt(1)
   \op
   GO
@@ -642,14 +650,15 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   AHEAD 2
   NEXT 6
 .Lw%=_taken\@:
-  v_readfirstlane_b32 s[rU], v[vF]
-  s_bfe_i32 s[rT], s[rW], s[rLo]
-  s_add_u32 s[rU], s[rU], 2
-  s_add_u32 s[rT], s[rT], s[rU]
+  v_add_u32 v[vD], 2, v[vF]           ; the address after the branch
+  v_bfe_i32 v[vA], v[vT], 16, 8
+  v_add_u32 v[vA], v[vD], v[vA]
+  ENTER vA
+  v_readfirstlane_b32 s[rU], v[vD]
+  v_readfirstlane_b32 s[rT], v[vA]
   s_cmp_gt_u32 s[rT], s[rLim]
   s_cbranch_scc1 .Lw%=_general
-  v_mov_b32 v[vF], s[rT]
-  ENTER
+  v_mov_b32 v[vF], v[vA]
   s_xor_b32 s[rU], s[rU], s[rT]
   s_lshr_b32 s[rU], s[rU], 8          ; SCC: another page
   s_cselect_b32 s[rU], 12, 9
@@ -661,20 +670,20 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_and_b32 s[rT], s[rV1], s[rV2]
   BRANCH_ \want, s_bitcmp1_b32 s[rT], 7
 .endm
-; A jump to the LDS address in rU, \dots charged.
+; A jump to the LDS address in rU, whose window has been read; \dots charged.
 .macro JUMP dots
   v_mov_b32 v[vF], s[rU]
-  ENTER
   PASS \dots, .Lw%=_exit
   ENTERED
 .endm
-; The LDS address of the 16-bit address in rT into rU; outside $8000-$FFF9 to
-; the general path.
-.macro TARGET
-  s_bitcmp0_b32 s[rT], 15
-  s_cbranch_scc1 .Lw%=_general
+; The window at the 16-bit address in \at, wherever that is; its LDS address
+; into rU from the scalar copy in rT.  Outside $8000-$FFF9 to the general path.
+.macro TARGET at, lo=0
+  v_bfe_u32 v[vD], v[\at], \lo, 15
+  ENTER vD, ROM
   s_sub_u32 s[rU], s[rT], 0x8000 - ROM
-  s_cmp_gt_u32 s[rU], s[rLim]
+  s_sub_u32 s[rT], s[rT], 0x8000
+  s_cmp_gt_u32 s[rT], LIM - ROM
   s_cbranch_scc1 .Lw%=_general
 .endm
 ; \add more than this instruction's address into \r.
@@ -755,7 +764,7 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_mov_b64 exec, -1
   s_branch .Lw%=_end
 .Lw%=_start:
-  ENTER
+  ENTER vF
   ENTERED
 .Lw%=_end:
   s_mov_b32 %0, s[rU]
@@ -799,6 +808,8 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_and_b32 s[rSP], s[rSP], s[rFF]
   s_bitset1_b32 s[rP], 2
   s_mov_b32 s[rU], s[rVec]
+  v_mov_b32 v[vA], s[rU]
+  ENTER vA
   JUMP 21
   R_INDX ORA, rA
   ILL
@@ -843,7 +854,7 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_cmp_eq_u32 s[rSP], 0
   s_cbranch_scc1 .Lw%=_general
   s_lshr_b32 s[rT], s[rW], 16
-  TARGET
+  TARGET vT, 16
   HERE rT, 2
   v_or_b32 v[vA], s[rSP], v[vRAM]
   v_mov_b32 v[vD], s[rT]
@@ -898,9 +909,8 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_waitcnt lgkmcnt(0)
   v_readfirstlane_b32 s[rM], v[vM]
   s_bfe_u32 s[rT], s[rM], 0x100008
-  TARGET
+  TARGET vM, 8
   v_mov_b32 v[vF], s[rU]
-  ENTER
   s_add_u32 s[rSP], s[rSP], 3
   s_and_b32 s[rP], s[rM], 0xCF
   UNPACK
@@ -926,7 +936,7 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 ; $4C JMP: to itself is the idle loop, left to the general path
   H
   s_lshr_b32 s[rT], s[rW], 16
-  TARGET
+  TARGET vT, 16
   v_readfirstlane_b32 s[rM], v[vF]
   s_cmp_eq_u32 s[rU], s[rM]
   s_cbranch_scc1 .Lw%=_general
@@ -954,9 +964,10 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   v_or_b32 v[vA], s[rSP], v[vRAM]
   ds_read_u16 v[vM], v[vA] offset:257
   s_waitcnt lgkmcnt(0)
+  v_add_u32 v[vM], 1, v[vM]
+  s_nop 0
   v_readfirstlane_b32 s[rT], v[vM]
-  s_add_u32 s[rT], s[rT], 1
-  TARGET
+  TARGET vM
   s_add_u32 s[rSP], s[rSP], 2
   JUMP 18
   R_INDX ADC, rA
@@ -1200,12 +1211,16 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_cmp_eq_u32 s[rT], 0x2007
   s_cbranch_scc1 .Lw%=_ppudata
   s_sub_u32 s[rU], s[rT], 0x4000
-  s_cmp_le_u32 s[rU], 0x15
+  s_cmp_le_u32 s[rU], 0x16
   s_cbranch_scc1 .Lw%=_apu
   s_cmp_eq_u32 s[rT], 0x2006
   s_cbranch_scc1 .Lw%=_ppuaddr
   s_cmp_eq_u32 s[rT], 0x2005
   s_cbranch_scc1 .Lw%=_ppuscroll
+  s_cmp_eq_u32 s[rT], 0x2001
+  s_cbranch_scc1 .Lw%=_ppumask
+  s_cmp_eq_u32 s[rT], 0x2000
+  s_cbranch_scc1 .Lw%=_ppuctrl
 .Lw%=_other:
   s_mov_b32 s[rR], s[rT]
   s_mov_b32 s[rK], 2
@@ -1214,13 +1229,16 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 .if SOLO == 0
   s_cbranch_vccnz .Lw%=_exit
 .endif
+  AIM
   GO
 .endm
 .macro OPENBUS
   s_andn2_b32 s[rIO], s[rIO], 0xFF
   s_or_b32 s[rIO], s[rIO], s[rM]
 .endm
-; $4000-$4015 but $4014: the byte kept for reads.
+; $4000-$4016 but $4014: the byte kept for reads; $4016 is the pads' strobe
+; too (high or on its way down it loads pad 1's buttons and clears the counts
+; of reads: flags bits 5 and 8-15, io bits 16-31).
 .Lw%=_apu:
   s_cmp_eq_u32 s[rU], 0x14
   s_cbranch_scc1 .Lw%=_other
@@ -1230,7 +1248,22 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   v_readfirstlane_b32 s[rCall], v[vP]
   v_readfirstlane_b32 s[rCall+1], v[vP+1]
   v_readfirstlane_b32 s[rR], v[vD]
+  s_cmp_lg_u32 s[rU], 0x16
   s_mul_i32 s[rU], s[rU], s[rR]
+  s_cbranch_scc1 .Lw%=_apubyte
+  s_bfe_u32 s[rT], s[rFL], 0x80008
+  s_lshl_b32 s[rT], s[rT], 16
+  s_and_b32 s[rR], s[rIO], 0xFFFF
+  s_or_b32 s[rT], s[rT], s[rR]
+  s_bfe_u32 s[rR], s[rFL], 0x10005
+  s_or_b32 s[rR], s[rR], s[rM]
+  s_bitcmp1_b32 s[rR], 0
+  s_cselect_b32 s[rIO], s[rT], s[rIO]
+  s_andn2_b32 s[rFL], s[rFL], 32
+  s_and_b32 s[rT], s[rM], 1
+  s_lshl_b32 s[rT], s[rT], 5
+  s_or_b32 s[rFL], s[rFL], s[rT]
+.Lw%=_apubyte:
   v_mov_b32 v[vD], s[rM]
   s_add_u32 s[rCall], s[rCall], s[rU]
   s_addc_u32 s[rCall+1], s[rCall+1], 0
@@ -1246,15 +1279,15 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   v_readfirstlane_b32 s[rR], v[vD]
   v_readfirstlane_b32 s[rCall], v[vP]
   v_readfirstlane_b32 s[rCall+1], v[vP+1]
-  s_and_b32 s[rW], s[rU], 0x3FFF
-  s_sub_u32 s[rW], s[rW], 0x2000
-  s_cmp_ge_u32 s[rW], 0x1F00
+  s_and_b32 s[rJ], s[rU], 0x3FFF
+  s_sub_u32 s[rJ], s[rJ], 0x2000
+  s_cmp_ge_u32 s[rJ], 0x1F00
   s_cbranch_scc1 .Lw%=_other
-  s_and_b32 s[rK], s[rW], s[rR]        ; mirroring: two masks (kWaveNt)
-  s_lshr_b32 s[rW], s[rW], 1
+  s_and_b32 s[rK], s[rJ], s[rR]        ; mirroring: two masks (kWaveNt)
+  s_lshr_b32 s[rJ], s[rJ], 1
   s_lshr_b32 s[rR], s[rR], 16
-  s_and_b32 s[rW], s[rW], s[rR]
-  s_or_b32 s[rK], s[rK], s[rW]
+  s_and_b32 s[rJ], s[rJ], s[rR]
+  s_or_b32 s[rK], s[rK], s[rJ]
   s_add_u32 s[rCall], s[rCall], s[rK]
   s_addc_u32 s[rCall+1], s[rCall+1], 0
   ds_read_u8 v[vM], v[vRG]
@@ -1291,6 +1324,35 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   v_mov_b32 v[vD], s[rU]
   ds_write_b16 v[vRG], v[vD] offset:18
   ds_write_b16 v[vRG], v[vD] offset:16
+  RESUME
+; PPUMASK.
+.Lw%=_ppumask:
+  OPENBUS
+  v_mov_b32 v[vD], s[rM]
+  ds_write_b8 v[vRG], v[vD] offset:1
+  RESUME
+; PPUCTRL: t's nametable too; turning NMI on during vblank raises one, which
+; the kernel takes.
+.Lw%=_ppuctrl:
+  ds_read_u8 v[vA], v[vRG]
+  ds_read_u16 v[vM], v[vRG] offset:18
+  s_waitcnt lgkmcnt(0)
+  v_readfirstlane_b32 s[rR], v[vA]
+  v_readfirstlane_b32 s[rU], v[vM]
+  s_andn2_b32 s[rR], s[rM], s[rR]
+  s_lshr_b32 s[rK], s[rIO], 8
+  s_and_b32 s[rR], s[rR], s[rK]
+  s_bitcmp1_b32 s[rR], 7
+  s_cbranch_scc1 .Lw%=_other
+  OPENBUS
+  s_and_b32 s[rU], s[rU], 0xF3FF
+  s_and_b32 s[rR], s[rM], 3
+  s_lshl_b32 s[rR], s[rR], 10
+  s_or_b32 s[rU], s[rU], s[rR]
+  v_mov_b32 v[vA], s[rM]
+  v_mov_b32 v[vD], s[rU]
+  ds_write_b8 v[vRG], v[vA]
+  ds_write_b16 v[vRG], v[vD] offset:18
   RESUME
 ; PPUSCROLL: x (fine x, t's coarse x), then y (t's coarse and fine y).
 .Lw%=_ppuscroll:
