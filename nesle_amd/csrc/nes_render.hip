@@ -18,8 +18,10 @@
 // then Pillow's BILINEAR resize to 84x84; the host computes its fixed-point
 // weights (nes_render.h).
 //
-// One workgroup of 256 threads renders one console in bands of 8 rows, in
-// three phases per band:
+// One workgroup of 256 threads renders one console (without the gray output:
+// a run of its bands, so that few consoles still fill the chip; 1 console 45
+// -> 6.4 us, 3,000 149 -> 140 us = 3.95 TB/s of RGB, where the vector unit
+// bounds it) in bands of 8 rows, in three phases per band:
 //  1. background: a thread owns 8 adjacent pixels of one row.  It reads the
 //     (at most two) tiles under them -- nametable byte, attribute, both
 //     pattern planes in one 16-bit read -- and turns each pixel's colour
@@ -32,9 +34,11 @@
 //     with an LDS atomic minimum -- the lowest OAM index wins, whatever the
 //     order;
 //  3. merge: a thread reads its 8 keys and replaces the background where a
-//     sprite key is present, all by byte permutes; it writes the full-size
-//     outputs as 8-byte runs (coalesced across the 32 threads of a row), and
-//     the band's gray levels feed the horizontal resample pass in LDS; the
+//     sprite key is present, all by byte permutes; it writes palette values
+//     as 8-byte runs (coalesced across the 32 threads of a row) and RGB as
+//     its wave's two rows in 16-byte words, gathered in LDS (24-byte runs per
+//     thread left every 64-byte line in three partial writes; 3,000 frames
+//     168 -> 149 us), and the band's gray levels feed the horizontal resample pass in LDS; the
 //     vertical pass runs once the intermediate rows an output row needs are
 //     complete.  Both passes sum an 8-input window with 4-way byte dot
 //     products over the weights' byte planes (exact), and run beside the
@@ -46,6 +50,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 #include "nes_layout.h"
 #include "nes_render.h"
@@ -56,6 +61,7 @@ namespace {
 constexpr std::uint32_t kThreads = 256;
 constexpr std::uint32_t kWaves = kThreads / 64;
 constexpr std::uint32_t kBand = 8;
+constexpr std::uint32_t kBands = 240 / kBand;   // 30: 1, 3, 5, 10 and 15 parts divide it
 // Horizontally resampled rows kept for the vertical pass.  An output row is
 // emitted after the first band that completes its input window; windows are
 // at most 7 rows and end within the band, so no emitted row reaches back more
@@ -199,19 +205,28 @@ __device__ __forceinline__ void merge(const uint4 k, std::uint32_t& d, std::uint
     g = (none & g) | (~none & gr);
 }
 
-__global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
+// LDS accesses of this wave before and after in program order, whatever their
+// types (the LDS unit keeps a wave's order; this holds the compiler to it).
+__device__ __forceinline__ void wave_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// kGray: the gray observation is among the outputs; its rows feed windows
+// that cross bands, so one workgroup draws the whole frame.  Without it a
+// frame is `gridDim.y` workgroups of consecutive bands.
+template <bool kGray>
+__device__ __forceinline__ void draw_frame(const RenderArgs& a) {
     __shared__ __attribute__((aligned(16))) std::uint16_t chr[4096];          // [512 tiles][8 rows]
     __shared__ __attribute__((aligned(16))) std::uint8_t rec[present::kMaxBytes];
     __shared__ __attribute__((aligned(16))) std::uint32_t line[kBand][256];   // sprite keys of the band
     // Gray rows of the last two bands (rows padded so a window's third dword
     // stays inside its row).
-    __shared__ __attribute__((aligned(16))) std::uint8_t gband[2][kBand][kGrayStride];
+    __shared__ __attribute__((aligned(16))) std::uint8_t gband[2][kGray ? kBand : 1][kGray ? kGrayStride : 16];
     // Horizontally resampled rows, column-major, the ring stored twice so an
     // output's window (kWindow rows from any ring position) is contiguous; a
     // column takes 9 dwords, so the 64 columns a wave touches fall in
     // distinct LDS banks.
-    __shared__ __attribute__((aligned(16))) std::uint8_t mid[render::kOut][kMidStride];
-    __shared__ __attribute__((aligned(16))) render::Staged tab;
+    __shared__ __attribute__((aligned(16))) std::uint8_t mid[kGray ? render::kOut : 1][kMidStride];
+    __shared__ __attribute__((aligned(16))) std::conditional_t<kGray, render::Vertical, uint4> vtab;
+    __shared__ __attribute__((aligned(16))) std::uint32_t rgbtab[64];
     __shared__ uint2 bgw[4];          // background palettes: display values, gray levels
     __shared__ uint2 spw[4];          // sprite palettes: palette values, gray levels
     __shared__ std::uint32_t bgo[4];  // background palettes: 1 where opaque
@@ -243,8 +258,11 @@ __global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
             reinterpret_cast<uint4*>(chr)[i] = make_uint4(perm(t.z, t.x, 0x05010400u), perm(t.z, t.x, 0x07030602u),
                                                           perm(t.w, t.y, 0x05010400u), perm(t.w, t.y, 0x07030602u));
         }
-        const uint4* t = reinterpret_cast<const uint4*>(&a.tables->s);
-        for (std::uint32_t i = tid; i < sizeof(render::Staged) / 16; i += kThreads) reinterpret_cast<uint4*>(&tab)[i] = t[i];
+        if constexpr (kGray) {
+            const uint4* t = reinterpret_cast<const uint4*>(&a.tables->s.v);
+            for (std::uint32_t i = tid; i < sizeof(render::Vertical) / 16; i += kThreads) reinterpret_cast<uint4*>(&vtab)[i] = t[i];
+        }
+        if (tid < 64) rgbtab[tid] = a.tables->s.rgb[tid];
         for (std::uint32_t i = tid; i < kBand * 256 / 4; i += kThreads)
             reinterpret_cast<uint4*>(line)[i] = make_uint4(kNoSprite, kNoSprite, kNoSprite, kNoSprite);
     }
@@ -307,23 +325,26 @@ __global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
     // read inside the row).
     const std::uint32_t h_rows = tid < 3 * render::kOut ? 1u : 0u;
     const std::uint32_t h_ox = tid % render::kOut, h_r0 = tid / render::kOut;
-    std::int32_t h_w[render::kWindow];
-    const render::Axis<render::kHTaps>& ht = a.tables->h;
-    const std::int32_t first = ht.lo[h_ox], taps = ht.n[h_ox];
-    const std::uint32_t h_lo = first + render::kWindow > 256 ? 256 - render::kWindow : first;
-    for (std::uint32_t j = 0; j < render::kWindow; ++j) {
-        const std::int32_t k = static_cast<std::int32_t>(j + h_lo) - first;   // tap index of input h_lo + j
-        h_w[j] = (k >= 0 && k < taps) ? ht.k[h_ox][k] : 0;
+    std::uint32_t h_lo = 0, h_k[6] = {};
+    if constexpr (kGray) {
+        std::int32_t h_w[render::kWindow];
+        const render::Axis<render::kHTaps>& ht = a.tables->h;
+        const std::int32_t first = ht.lo[h_ox], taps = ht.n[h_ox];
+        h_lo = first + render::kWindow > 256 ? 256 - render::kWindow : first;
+        for (std::uint32_t j = 0; j < render::kWindow; ++j) {
+            const std::int32_t k = static_cast<std::int32_t>(j + h_lo) - first;   // tap index of input h_lo + j
+            h_w[j] = (k >= 0 && k < taps) ? ht.k[h_ox][k] : 0;
+        }
+        render::pack_weights(h_w, h_k);
     }
-    std::uint32_t h_k[6];
-    render::pack_weights(h_w, h_k);
     // Band k is drawn in iteration k (background and sprites, then the merge)
     // while iteration k + 1 resamples it (horizontal pass beside band k + 1's
     // background and sprites, vertical pass beside its merge): two barriers a
     // band.  The gray rows of a band alternate between two buffers.
-    constexpr std::uint32_t kBands = 240 / kBand;
-    for (std::uint32_t band = 0; band <= kBands; ++band) {
-        const bool draw = band < kBands, resample = a.gray && band > 0;
+    const std::uint32_t bands = kGray ? kBands : kBands / gridDim.y, band0 = kGray ? 0 : blockIdx.y * bands;
+    const std::uint32_t band1 = band0 + bands;
+    for (std::uint32_t band = band0; band < band1 + (kGray ? 1 : 0); ++band) {
+        const bool draw = !kGray || band < band1, resample = kGray && band > 0;
         const std::uint32_t y0 = band * kBand, y = y0 + r;
         std::uint32_t d[2], g[2];
         if (draw) {
@@ -393,7 +414,7 @@ __global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
                 }
             }
         }
-        if (resample && h_rows != 0) {   // horizontal pass of the previous band: column h_ox of rows h_r0, +3, +6
+        if constexpr (kGray) if (resample && h_rows != 0) {   // horizontal pass of the previous band: column h_ox of rows h_r0, +3, +6
             for (std::uint32_t rr = h_r0; rr < kBand; rr += 3) {
                 const uint2 w = bytes8(gband[(band - 1) & 1][rr], h_lo);
                 const std::uint32_t slot = (y0 - kBand + rr) % kRing;
@@ -407,34 +428,45 @@ __global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
                 uint4* keys = reinterpret_cast<uint4*>(&line[r][x0]);
                 merge(keys[0], d[0], g[0]);
                 merge(keys[1], d[1], g[1]);
-                keys[0] = keys[1] = make_uint4(kNoSprite, kNoSprite, kNoSprite, kNoSprite);
+                if (!a.rgb) keys[0] = keys[1] = make_uint4(kNoSprite, kNoSprite, kNoSprite, kNoSprite);
             }
             const std::size_t pix = static_cast<std::size_t>(env) * 240 * 256 + y * 256 + x0;
             if (a.palette) *reinterpret_cast<uint2*>(a.palette + pix) = make_uint2(d[0], d[1]);
             if (a.rgb) {   // 8 pixels' RGB: one palette word per pixel, packed by 3 permutes per 4 pixels
                 std::uint32_t c[8], w[6];
-                for (std::uint32_t i = 0; i < 8; ++i) c[i] = tab.rgb[byte_of(d, i)];
+                for (std::uint32_t i = 0; i < 8; ++i) c[i] = rgbtab[byte_of(d, i)];
                 for (std::uint32_t h = 0; h < 2; ++h) {
                     const std::uint32_t* q = c + 4 * h;
                     w[3 * h] = perm(q[1], q[0], 0x04020100u);       // R0 G0 B0 R1
                     w[3 * h + 1] = perm(q[2], q[1], 0x05040201u);   // G1 B1 R2 G2
                     w[3 * h + 2] = perm(q[3], q[2], 0x06050402u);   // B2 R3 G3 B3
                 }
-                uint2* o = reinterpret_cast<uint2*>(a.rgb + pix * 3);
+                // The wave's two rows are 1,536 adjacent bytes of the frame:
+                // gathered where its sprite keys were and stored as 16-byte
+                // words in order.
+                uint4* out = reinterpret_cast<uint4*>(a.rgb + (static_cast<std::size_t>(env) * 240 + y0 + 2 * wave) * 768);
+                uint4* rows = reinterpret_cast<uint4*>(&line[2 * wave][0]);
+                uint2* o = reinterpret_cast<uint2*>(rows) + 3 * lane;
+                wave_order();
                 o[0] = make_uint2(w[0], w[1]);
                 o[1] = make_uint2(w[2], w[3]);
                 o[2] = make_uint2(w[4], w[5]);
+                wave_order();
+                out[lane] = rows[lane];
+                if (lane < 32) out[64 + lane] = rows[64 + lane];
+                wave_order();
+                rows[2 * lane] = rows[2 * lane + 1] = make_uint4(kNoSprite, kNoSprite, kNoSprite, kNoSprite);
             }
-            if (a.gray) *reinterpret_cast<uint2*>(&gband[band & 1][r][x0]) = make_uint2(g[0], g[1]);
+            if constexpr (kGray) *reinterpret_cast<uint2*>(&gband[band & 1][r][x0]) = make_uint2(g[0], g[1]);
         }
-        if (resample) {   // vertical pass of every output row whose window the previous band completed
+        if constexpr (kGray) if (resample) {   // vertical pass of every output row whose window the previous band completed
             std::uint32_t end = next_oy;
-            while (end < render::kOut && static_cast<std::uint32_t>(tab.v.lo[end] + tab.v.n[end]) <= y0)
+            while (end < render::kOut && static_cast<std::uint32_t>(vtab.lo[end] + vtab.n[end]) <= y0)
                 ++end;
             std::uint8_t* out = a.gray + static_cast<std::size_t>(env) * render::kOut * render::kOut;
             for (std::uint32_t oy = next_oy + h_r0; h_rows != 0 && oy < end; oy += 3) {
-                const uint2 w = bytes8(mid[h_ox], tab.v.lo[oy] % kRing);
-                const uint4* k = reinterpret_cast<const uint4*>(tab.v.kb[oy]);
+                const uint2 w = bytes8(mid[h_ox], vtab.lo[oy] % kRing);
+                const uint4* k = reinterpret_cast<const uint4*>(vtab.kb[oy]);
                 const uint4 k0 = k[0], k1 = k[1];
                 const std::uint32_t kv[6] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y};
                 out[oy * render::kOut + h_ox] = static_cast<std::uint8_t>(clip8(window8(w, kv)));
@@ -444,6 +476,9 @@ __global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) {
         __syncthreads();
     }
 }
+
+__global__ void __launch_bounds__(kThreads) render_kernel(RenderArgs a) { draw_frame<true>(a); }
+__global__ void __launch_bounds__(kThreads) frame_kernel(RenderArgs a) { draw_frame<false>(a); }
 
 }  // namespace
 
@@ -532,7 +567,25 @@ Tables make_tables() {
 
 hipError_t launch_render(const RenderArgs& a, hipStream_t stream) {
     if (a.n == 0) return hipSuccess;
-    render_kernel<<<dim3(a.n), dim3(kThreads), 0, stream>>>(a);
+    if (a.gray != nullptr) {
+        render_kernel<<<dim3(a.n), dim3(kThreads), 0, stream>>>(a);
+    } else {
+        // Parts of a frame: as few as give the chip's 1,792 resident
+        // workgroups (7 a compute unit) two thirds of their number, at least
+        // 3, so that the last of them do not run on an idle chip.  Measured,
+        // us for 1, 2, 3, 5, 10, 15 parts: 1 console 45, 25, 18, 12, 7.9,
+        // 6.4; 64: 48, 26, 19, 14, 11, 9.7; 256: 48, 31, 25, 21.5, 22, 22.5;
+        // 1,000: 66, 60, 57, 57, 60, 65; 3,000: 149, 141, 140, 142, 160, 178
+        // (each part stages the pattern tables again).
+        constexpr std::uint32_t kTarget = 1200;
+        std::uint32_t parts = 15;
+        for (const std::uint32_t p : {10u, 5u, 3u})
+            if (static_cast<std::uint64_t>(a.n) * p >= kTarget) parts = p;
+        // Where every part gathers the console's CHR RAM (live state), more
+        // than one only while all of them are resident.
+        if (a.cpu_rules != 0 && a.chr_size == 0 && parts != 15) parts = 1;
+        frame_kernel<<<dim3(a.n, parts), dim3(kThreads), 0, stream>>>(a);
+    }
     return hipGetLastError();
 }
 

@@ -411,3 +411,28 @@ def test_live_frames_of_random_states_with_chr_ram():
     assert np.array_equal(b.host(abi.VIEW_PRESENT), before)
     # The batched rules still draw the snapshot, with CHR RAM read as 0.
     _check(b, oracles, "snapshot after a live render")
+
+
+# Without the gray output a frame is drawn in 15, 10, 5 or 3 parts, by the
+# batch; live state of a CHR RAM cart in 15 or one.
+@pytest.mark.parametrize("live", [False, True])
+@pytest.mark.parametrize("num_envs", [1, 79, 80, 119, 120, 239, 240, 401])
+def test_frames_drawn_in_parts(num_envs, live):
+    rom = _rom(7, mirroring="horizontal", chr_ram=live)
+    say(f"[gpu] frames in parts: N={num_envs} live={live}")
+    b = abi.Batch(rom, num_envs, frameskip=3)
+    sample = {0, num_envs // 2, num_envs - 1}
+    oracles = {e: O.Oracle(rom) for e in sample}
+    for k in range(3):
+        _step_all(b, oracles, 11, k, 3)
+    flag = abi.FRAME_LIVE if live else 0
+    b.render(abi.FRAME_RGB | abi.FRAME_GRAY84 | flag)
+    whole = b.host(abi.VIEW_FRAME_RGB).copy()   # one workgroup a frame
+    if not live:
+        _check(b, oracles, "in parts", abi.FRAME_RGB | abi.FRAME_PALETTE)
+    b.render(abi.FRAME_RGB | abi.FRAME_PALETTE | flag)
+    rgb, pal = b.host(abi.VIEW_FRAME_RGB), b.host(abi.VIEW_FRAME_PALETTE)
+    assert np.array_equal(rgb, whole)
+    assert np.array_equal(rgb, O.palette_rgb()[pal])
+    b.render(abi.FRAME_PALETTE | flag)
+    assert np.array_equal(b.host(abi.VIEW_FRAME_PALETTE), pal)
