@@ -195,6 +195,10 @@ int nesle_get_view(nesle_batch* b, int kind, nesle_view* out);
  * 841-852, 904-915). */
 int nesle_copy_to_host(nesle_batch* b, int kind, void* dst, size_t bytes);
 
+/* The same for `count` views with one wait: dsts[i] receives view kinds[i],
+ * bytes[i] long.  Not for NESLE_VIEW_OAM. */
+int nesle_copy_views(nesle_batch* b, const int* kinds, void* const* dsts, const size_t* bytes, uint32_t count);
+
 /* Draw every console's frame from its presentation snapshot (frozen at the
  * last vblank; seeded from live state by full resets and state loads) into
  * the device buffers selected by `outputs` (NESLE_FRAME_*), allocated on

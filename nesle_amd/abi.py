@@ -140,6 +140,8 @@ def lib():
         "nesle_step": (ctypes.c_int, [vp, ctypes.c_int, ctypes.c_int]),
         "nesle_get_view": (ctypes.c_int, [vp, ctypes.c_int, ctypes.POINTER(View)]),
         "nesle_copy_to_host": (ctypes.c_int, [vp, ctypes.c_int, vp, ctypes.c_size_t]),
+        "nesle_copy_views": (ctypes.c_int, [vp, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(vp),
+                                            ctypes.POINTER(ctypes.c_size_t), ctypes.c_uint32]),
         "nesle_render": (ctypes.c_int, [vp, ctypes.c_uint32]),
         "nesle_save_state": (ctypes.c_int, [vp, ctypes.c_uint32, _U8P]),
         "nesle_load_state": (ctypes.c_int, [vp, ctypes.c_char_p, ctypes.c_size_t, _U8P]),

@@ -326,12 +326,24 @@ public:
         set_host_actions(actions);
         check(nesle_step(h_, 0, 0));
         if (frames_ && (render_frame || copy_obs)) check(nesle_render(h_, NESLE_FRAME_RGB));
+        // Everything comes back with one wait.
+        const py::ssize_t n = n_;
+        py::array_t<float> rewards({n});
+        py::array_t<std::uint8_t> dones({n});
+        int kinds[3] = {NESLE_VIEW_REWARDS, NESLE_VIEW_DONES, frames_ ? NESLE_VIEW_FRAME_RGB : NESLE_VIEW_RAM};
+        void* to[3] = {rewards.mutable_data(), dones.mutable_data(), nullptr};
+        std::size_t bytes[3] = {static_cast<std::size_t>(rewards.nbytes()), static_cast<std::size_t>(dones.nbytes()), 0};
         py::dict out;
         if (copy_obs) {
-            out["obs"] = frames_ ? host<std::uint8_t>(NESLE_VIEW_FRAME_RGB, {py::ssize_t(n_), 240, 256, 3}) : ram();
+            py::array_t<std::uint8_t> obs(frames_ ? std::vector<py::ssize_t>{n, 240, 256, 3}
+                                                  : std::vector<py::ssize_t>{n, 2048});
+            to[2] = obs.mutable_data();
+            bytes[2] = static_cast<std::size_t>(obs.nbytes());
+            out["obs"] = obs;
         }
-        out["rewards"] = host<float>(NESLE_VIEW_REWARDS, {py::ssize_t(n_)});
-        out["dones"] = host<std::uint8_t>(NESLE_VIEW_DONES, {py::ssize_t(n_)});
+        check(nesle_copy_views(h_, kinds, to, bytes, copy_obs ? 3 : 2));
+        out["rewards"] = rewards;
+        out["dones"] = dones;
         return out;
     }
 

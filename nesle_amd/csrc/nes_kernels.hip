@@ -233,6 +233,17 @@ __global__ void __launch_bounds__(kBlock) zero_u64_kernel(unsigned long long* p,
     if (i < n) p[i] = 0ull;
 }
 
+// Buffer blockIdx.y of a StageCopy, in 16-byte words and a tail of bytes.
+__global__ void __launch_bounds__(kBlock) stage_copy_kernel(StageCopy c) {
+    const std::uint32_t bytes = c.bytes[blockIdx.y], words = bytes / 16;
+    const std::uint8_t* src = c.src[blockIdx.y];
+    std::uint8_t* dst = c.dst[blockIdx.y];
+    const std::uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    for (std::uint32_t i = t; i < words; i += gridDim.x * kBlock)
+        reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < bytes % 16) dst[16 * words + threadIdx.x] = src[16 * words + threadIdx.x];
+}
+
 __global__ void __launch_bounds__(kBlock) seed_kernel(DeviceState s) {
     const std::uint32_t env = blockIdx.x * kBlock + threadIdx.x;
     if (env < s.n) reward_seed(s, env, GlobalRam{s, env});
@@ -390,6 +401,19 @@ hipError_t launch_ram_obs(const DeviceState& s, std::uint8_t* obs, hipStream_t s
 
 hipError_t launch_actions_i64(std::uint8_t* dst, const long long* src, std::uint32_t n, hipStream_t stream) {
     actions_i64_kernel<<<dim3(blocks_for(n)), dim3(kBlock), 0, stream>>>(dst, src, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_stage_copy(const StageCopy& c, std::uint32_t count, hipStream_t stream) {
+    std::uint32_t most = 0;
+    for (std::uint32_t i = 0; i < count; ++i) {
+        if ((reinterpret_cast<std::uintptr_t>(c.src[i]) | reinterpret_cast<std::uintptr_t>(c.dst[i])) % 16 != 0)
+            return hipErrorInvalidValue;
+        most = c.bytes[i] > most ? c.bytes[i] : most;
+    }
+    if (most == 0 || count > kStageCopies) return count > kStageCopies ? hipErrorInvalidValue : hipSuccess;
+    const std::uint32_t blocks = (most / 16 + kBlock - 1) / kBlock;
+    stage_copy_kernel<<<dim3(blocks == 0 ? 1 : blocks, count), dim3(kBlock), 0, stream>>>(c);
     return hipGetLastError();
 }
 

@@ -29,6 +29,15 @@ hipError_t launch_poke_ram(const DeviceState& s, std::uint32_t addr, std::uint32
 hipError_t launch_poke_ram_envs(const DeviceState& s, std::uint32_t addr, const std::uint8_t* values,
                                 hipStream_t stream);
 hipError_t launch_seed_baselines(const DeviceState& s, hipStream_t stream);
+// Up to kStageCopies buffers copied by one kernel, device memory or pinned
+// host memory on either side; sources and destinations on 16-byte boundaries.
+constexpr std::uint32_t kStageCopies = 3;
+struct StageCopy {
+    const std::uint8_t* src[kStageCopies];
+    std::uint8_t* dst[kStageCopies];
+    std::uint32_t bytes[kStageCopies];
+};
+hipError_t launch_stage_copy(const StageCopy& c, std::uint32_t count, hipStream_t stream);
 // n 64-bit words set to zero by a kernel (graph-capturable, unlike a memset).
 hipError_t launch_zero_u64(unsigned long long* p, std::uint32_t n, hipStream_t stream);
 // Presentation snapshot (and pre-render latch) from live state, masked.

@@ -189,3 +189,29 @@ def test_ram_device_matches_oracle_after_steps():
     ram = torch.utils.dlpack.from_dlpack(batch.ram_device()).cpu().numpy()
     for e, o in enumerate(oracles):
         assert np.array_equal(ram[e], o.save()[O.OFF["ram"]:O.OFF["ram"] + 2048])
+
+
+# Actions in and views out through pinned memory up to 1 MiB, straight above:
+# a batch of each, on its own stream, its pads overwritten right after the
+# call that took them.
+@pytest.mark.parametrize("num_envs,frames", [(1, True), (5, True), (6, True), (63, False), (511, False), (513, False)])
+def test_host_step_matches_device_step(num_envs, frames):
+    import torch
+
+    core = _core()
+    rom = synthrom.make_rom(5).rom
+    a = core.CudaBatch(num_envs, 2, rom, frames=frames)
+    b = core.CudaBatch(num_envs, 2, rom, frames=frames)
+    stream = torch.cuda.Stream()
+    a.set_stream(stream.cuda_stream)
+    for k in range(4):
+        pads = synthrom.action_masks(3, num_envs, k)
+        want = torch.from_numpy(pads.copy()).cuda()
+        mine = pads.copy()
+        got = a.step(mine, render_frame=False, copy_obs=True)
+        mine[:] = 0xFF
+        b.step_device(want, auto_reset=False, synchronize=True)
+        assert np.array_equal(a.ram(), torch.from_dlpack(b.ram_device()).cpu().numpy())
+        assert np.array_equal(got["rewards"], torch.from_dlpack(b.rewards_device()).cpu().numpy())
+        assert np.array_equal(got["dones"], torch.from_dlpack(b.last_done_device()).cpu().numpy())
+        assert np.array_equal(got["obs"], b.render() if frames else b.ram())
