@@ -434,16 +434,19 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   .endr
 .endm
 ; Reads.
+.macro LD_IMM r
+  H
+  s_bfe_u32 s[\r], s[rW], s[rLo]
+  AHEAD 2
+  s_mov_b32 s[rNZ], s[\r]
+  NEXT 6
+.endm
 .macro R_IMM op, r
   H
   s_bfe_u32 s[rM], s[rW], s[rLo]
   AHEAD 2
   IMM_\op \r
   NEXT 6
-.endm
-.macro IMM_LD r
-  s_mov_b32 s[\r], s[rM]
-  s_mov_b32 s[rNZ], s[rM]
 .endm
 .macro IMM_ORA r
   s_or_b32 s[rA], s[rA], s[rM]
@@ -651,14 +654,12 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   NEXT 6
 .Lw%=_taken\@:
   v_add_u32 v[vD], 2, v[vF]           ; the address after the branch
-  v_bfe_i32 v[vA], v[vT], 16, 8
-  v_add_u32 v[vA], v[vD], v[vA]
-  ENTER vA
+  v_add_u32_sdwa v[vF], v[vD], sext(v[vT]) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2
+  ENTER vF
   v_readfirstlane_b32 s[rU], v[vD]
-  v_readfirstlane_b32 s[rT], v[vA]
+  v_readfirstlane_b32 s[rT], v[vF]
   s_cmp_gt_u32 s[rT], s[rLim]
-  s_cbranch_scc1 .Lw%=_general
-  v_mov_b32 v[vF], v[vA]
+  s_cbranch_scc1 .Lw%=_back
   s_xor_b32 s[rU], s[rU], s[rT]
   s_lshr_b32 s[rU], s[rU], 8          ; SCC: another page
   s_cselect_b32 s[rU], 12, 9
@@ -1035,16 +1036,16 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   W_ABSI rA, rX
   ILL 2
 ; $A0
-  R_IMM LD, rY
+  LD_IMM rY
   R_INDX LD, rA
-  R_IMM LD, rX
+  LD_IMM rX
   ILL
   R_ZP LD, rY
   R_ZP LD, rA
   R_ZP LD, rX
   ILL
   T_ rY, rA
-  R_IMM LD, rA
+  LD_IMM rA
   T_ rX, rA
   ILL
   R_ABS LD, rY
@@ -1390,6 +1391,9 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
 .Lw%=_exit:
   s_mov_b32 s[rK], 1
   s_branch .Lw%=_leave
+; A taken branch that leaves the image: the PC back at it, from vD past it.
+.Lw%=_back:
+  v_subrev_u32 v[vF], 2, v[vD]
 .Lw%=_general:
   s_mov_b32 s[rK], 0
 .Lw%=_leave:
