@@ -92,15 +92,21 @@ def profile_figure(key: str, num_envs: int) -> float | None:
     return None
 
 
+# Largest batch the one-console-per-wave step kernels take.
+ONE_PER_WAVE_MAX = 32768
+
+
 def size_figures(run: dict, num_envs: int) -> dict:
     """Throughput and roofline fractions of one batch size: NES frames/s,
     algorithmic and measured (rocprofv3, committed summary) HBM bytes per
     kernel time against the 8 TB/s peak, and the VALU pipe's busy fraction."""
     kernel_s = run["kernel_ms_per_launch"] / 1000.0
     algo = num_envs * B_STEP / kernel_s / 1e9
-    traffic = profile_figure("traffic_bytes_per_launch", num_envs)
+    # The summary's counters are the lane kernel's.
+    counted = num_envs > ONE_PER_WAVE_MAX
+    traffic = profile_figure("traffic_bytes_per_launch", num_envs) if counted else None
     measured = traffic / kernel_s / 1e9 if traffic else None
-    lane_ops = profile_figure("valu_lane_ops_per_launch", num_envs)
+    lane_ops = profile_figure("valu_lane_ops_per_launch", num_envs) if counted else None
     lanes = consoles_per_wave(num_envs)
     return {
         "num_envs": num_envs,
@@ -112,7 +118,7 @@ def size_figures(run: dict, num_envs: int) -> dict:
         "hbm_algorithmic_frac": algo / HBM_PEAK_GBS,
         "hbm_measured_gbs": measured,
         "hbm_measured_frac": measured / HBM_PEAK_GBS if measured else None,
-        "valu_busy_frac": profile_figure("valu_busy", num_envs),
+        "valu_busy_frac": profile_figure("valu_busy", num_envs) if counted else None,
         "valu_lane_ops_frac": lane_ops / kernel_s / VALU_PEAK_LANE_OPS if lane_ops else None,
         "consoles_per_wave": lanes,
         # Lanes without a console run the datapath on a dummy block: only
@@ -123,8 +129,11 @@ def size_figures(run: dict, num_envs: int) -> dict:
 
 
 def consoles_per_wave(num_envs: int) -> int:
-    """Consoles per wave64 of the step kernel's launch: the smallest power of
-    two L (at most 64) with 1,024 waves x L >= num_envs (one wave per SIMD)."""
+    """Consoles per wave64 of the step kernel's launch: one up to
+    ONE_PER_WAVE_MAX consoles; above, the smallest power of two L (at most 64)
+    with 1,024 waves x L >= num_envs (one wave per SIMD)."""
+    if num_envs <= ONE_PER_WAVE_MAX:
+        return 1
     lanes = 1
     while lanes < 64 and 1024 * lanes < num_envs:
         lanes *= 2
