@@ -436,10 +436,26 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
 
 // Waves per workgroup: as few as keep the batch within one workgroup per CU,
 // so that every CU has its share; more than 16 a CU become two workgroups.
+// Of those, 12 waves where the chip's 512 resident workgroups then take no
+// round more than with 16, as six waves per SIMD end sooner than eight and a
+// few workgroups left for a last round run longer beside a full one.  ms per
+// step with 16 -> 12 waves: one round, 4,097 consoles 3.34 -> 3.03, 6,144 3.35
+// -> 2.99 (frame-skip 1 0.97 -> 0.81, a game that idles 1.18 -> 1.02); a second
+// round of at most one workgroup per CU, 8,200 6.23 -> 5.64, 9,200 6.43 ->
+// 5.40 (beyond it 9,400 6.08 -> 6.00, but 1.53 -> 1.66 at frame-skip 1); a
+// third, 16,400 9.10 -> 8.64, 18,200 8.88 -> 8.60, but 2.32 -> 2.39 at
+// frame-skip 1, where loads and stores weigh more: only from frame-skip 4.
 hipError_t NESLE_WAVE_LAUNCH(const DeviceState& s, std::uint32_t frameskip, hipStream_t stream) {
-    std::uint32_t waves = (s.n + 255) / 256;
+    constexpr std::uint32_t kCus = 256, kResident = 2 * kCus, kFewer = 12;
+    std::uint32_t waves = (s.n + kCus - 1) / kCus;
     if (waves > 2) waves = (waves + 3) & ~3u;
-    if (waves > kWaveMaxWaves) waves = kWaveMaxWaves;
+    if (waves > kWaveMaxWaves) {
+        const std::uint32_t round = kResident * kWaveMaxWaves, fewer = (s.n + kFewer - 1) / kFewer;
+        const bool pays = s.n <= round ? fewer <= kResident
+                          : s.n <= 2 * round ? fewer <= kResident + kCus
+                                             : fewer <= 3 * kResident && frameskip >= 4;
+        waves = pays ? kFewer : kWaveMaxWaves;
+    }
     NESLE_WAVE_KERNEL<<<dim3((s.n + waves - 1) / waves), dim3(64 * waves), 0, stream>>>(s, frameskip);
     return hipGetLastError();
 }

@@ -101,6 +101,15 @@ def test_sizes_agree_with_the_lane_kernel(n, frameskip):
     twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 77)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,frameskip", [(6143, 2), (6145, 1), (9205, 2), (9217, 1), (18421, 4)])
+def test_workgroups_of_twelve_waves_agree_with_the_lane_kernel(n, frameskip):
+    """Both sides of the sizes that take 12 waves per workgroup instead of 16,
+    ragged: one, one and a half and three rounds of workgroups on the chip."""
+    say(f"[gpu] wave kernel, 12 or 16 waves: N={n} fs={frameskip}")
+    twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 78)
+
+
 def poll_rom() -> bytes:
     """Reads of $2007 and $4015 and PRG RAM traffic without end: nearly every
     instruction takes the general path."""
