@@ -5,11 +5,11 @@
 // emulated instruction however few consoles it serves: at 4,096 consoles 60
 // of 64 lanes idle, and a single console takes as long as 8,192.  Here a wave
 // runs one console on the scalar unit, each opcode by its own code
-// (nes_wave.h), about 190 cycles per instruction alone on a SIMD and 32 per
+// (nes_wave.h), about 165 cycles per instruction alone on a SIMD and 30 per
 // SIMD with eight waves on it.  Frame-skip 4, the workload ROM, ms per launch
 // (lane kernel -> this one): 1 console 13.0 -> 2.13, 1,000 13.4 -> 2.46,
-// 4,096 13.8 -> 2.74, 8,192 14.1 -> 3.43, 16,384 16.7 -> 6.66, 32,768
-// 17.3 -> 13.2.
+// 4,096 13.8 -> 2.73, 8,192 14.1 -> 3.37, 16,384 16.7 -> 6.51, 32,768
+// 17.3 -> 12.9.
 //
 // What the block of assembly leaves to the general path here -- I/O and PRG
 // RAM, NMI entry, code outside PRG ROM, PPU events, OAM DMA, frame capture --

@@ -53,8 +53,8 @@
 //   SOLO = 1, few waves per SIMD (the wave's own time bounds): an event
 //   selects another table, all of whose entries leave the block, instead of
 //   branching, in the shadow of the operand's read.
-//   SOLO = 0, many waves (both units bound, at 6.2 scalar and 6.5 vector
-//   instructions per emulated one, 32 cycles per SIMD): the countdown is a
+//   SOLO = 0, many waves (both units bound, at 6.1 scalar and 6.3 vector
+//   instructions per emulated one, 30 cycles per SIMD): the countdown is a
 //   vector register and the event a branch on its borrow.
 // At 1,000 consoles the first takes 2.47 ms per 4-frame step, the second
 // 2.80; at 8,192 3.92 and 3.43.  A store that leaves the block costs 200
