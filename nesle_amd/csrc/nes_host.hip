@@ -17,9 +17,9 @@
 #include <vector>
 
 #include "../../include/nesle_hip.h"
+#include "nes_choice.h"
 #include "nes_launch.h"
 #include "nes_layout.h"
-#include "nes_micro.h"
 #include "nes_render.h"
 
 using nesle::DeviceState;
@@ -599,28 +599,6 @@ void check_config(const nesle_config* cfg) {
     if (cfg->reward_kind > NESLE_REWARD_XDELTA) throw InvalidArgument("unknown reward_kind");
 }
 
-// Whether straight-line flow into the vectors ($FFFA-$FFFF) meets no
-// instruction whose bytes run past $FFFF (they would wrap to RAM).  Any
-// instruction may start at $FFF8 or $FFF9; from there on what falls into what
-// is given by the image.  (Jumps to the vectors are not flow in this sense:
-// the step kernel runs those instructions one at a time.)
-bool closed_end(const std::vector<std::uint8_t>& prg) {
-    constexpr std::uint32_t kTail = 8;
-    bool reached[kTail] = {true, true};
-    for (std::uint32_t o = 0; o < kTail; ++o) {
-        if (!reached[o]) continue;
-        const std::uint8_t op = prg[prg.size() - kTail + o];
-        const auto& w = nesle::mc::kTableFull.e[op];
-        if (w.d[14] & nesle::mc::kIllegal) continue;
-        const std::uint32_t next = o + ((w.d[0] >> 12) & 3);
-        if (next > kTail) return false;
-        // JMP, JSR, RTS, RTI and BRK do not go on to the next instruction.
-        const bool leaves = w.d[9] != 0 || w.d[10] != 0 || w.d[11] != 0 || (w.d[14] & nesle::mc::kJmpInd) != 0;
-        if (!leaves && next < kTail) reached[next] = true;
-    }
-    return true;
-}
-
 // Allocate and power on a batch for `b->rom` (parsed and checked by the caller).
 void open_batch(nesle_batch* b, const nesle_config* cfg) {
     int dev = cfg->device;
@@ -642,7 +620,7 @@ void open_batch(nesle_batch* b, const nesle_config* cfg) {
     s.done_addr = b->cfg.done_addr & 0x7FF;
     s.clip = b->cfg.clip;
     s.time_penalty = b->cfg.time_penalty;
-    b->closed_end = closed_end(b->rom.prg);
+    b->closed_end = nesle::closed_end(b->rom.prg.data(), b->rom.prg.size());
     void* general = nullptr;
     hip_check(hipHostMalloc(&general, sizeof(std::uint32_t) * nesle::kGeneralSlots, hipHostMallocMapped),
               "hipHostMalloc general-path reports");

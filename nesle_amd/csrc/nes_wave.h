@@ -32,7 +32,7 @@
 // bits 16-31 (vT holds it too, for the vector unit).  The PC is an LDS
 // address in vF.  No instruction checks whether its successor lies past the
 // PRG image: the host runs only images here whose straight-line flow cannot
-// get there in the middle of an instruction (closed_end, nes_host.hip), 128
+// get there in the middle of an instruction (closed_end, nes_choice.h), 128
 // bytes of an illegal opcode stand on either side of the image (a branch
 // leaves it downwards by at most that), and jumps test their target.
 //

@@ -158,6 +158,10 @@ def vector_rom(irq: int, flow: list[int]) -> bytes:
     (0xADEA, [0x4C, 0xFF, 0xFF]),    # the same instruction entered by a jump
     (0xEAEA, [0x18, 0x90, 0x06]),    # a branch over the end
     (0x9090, [0x18, 0x90, 0x02]),    # a branch to the vectors
+    # Three bytes at $FFF7 fall into $FFFA, past operands that are no opcodes.
+    (0xADEA, [0xEA, 0xEA, 0xAD, 0x02, 0x03]),
+    (0xADEA, [0xEA, 0xEA, 0x8D, 0x02, 0x03]),
+    (0xEA8D, [0xEA, 0xEA, 0xAD, 0x02, 0x03]),
 ])
 def test_flow_over_the_vectors_matches_oracle(irq, flow):
     rom = vector_rom(irq, flow)

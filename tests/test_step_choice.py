@@ -1,0 +1,92 @@
+"""Which kernel steps a batch (nesle_amd/csrc/nes_choice.h), compiled alone and
+without a GPU: the test for images whose flow runs past $FFFF."""
+
+from __future__ import annotations
+
+import ctypes
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from nesle_amd import build
+
+CXX = os.environ.get("CXX") or shutil.which("g++") or shutil.which("clang++")
+pytestmark = pytest.mark.skipif(CXX is None, reason="no host C++ compiler")
+
+SHIM = r"""
+#include "nes_choice.h"
+using namespace nesle;
+extern "C" int t_closed_end(const std::uint8_t* prg, std::size_t size) { return closed_end(prg, size); }
+"""
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    work = tmp_path_factory.mktemp("choice")
+    (work / "shim.cpp").write_text(SHIM)
+    subprocess.run([CXX, "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{build.CSRC}", str(work / "shim.cpp"), "-o",
+                    str(work / "shim.so")], check=True, capture_output=True, text=True)
+    L = ctypes.CDLL(str(work / "shim.so"))
+    L.t_closed_end.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+    return L
+
+
+# Lengths of the official opcodes, one row per high digit (0: illegal), and
+# those that do not go on to the next instruction (BRK, JSR, RTI, JMP, RTS).
+LENGTHS = [int(c) for row in (
+    "1200022012100330", "2200022013000330", "3200222012103330", "2200022013000330",
+    "1200022012103330", "2200022013000330", "1200022012103330", "2200022013000330",
+    "0200222010103330", "2200222013100300", "2220222012103330", "2200222013103330",
+    "2200222012103330", "2200022013000330", "2200222012103330", "2200022013000330") for c in row]
+LEAVES = {0x00, 0x20, 0x40, 0x4C, 0x60, 0x6C}
+
+
+def runs_past_the_end(prg: bytes) -> bool:
+    """Walks the flow from every start in the last bytes below $FFFA."""
+    for at in range(len(prg) - 26, len(prg) - 6):
+        while at < len(prg):
+            op = prg[at]
+            if LENGTHS[op] == 0:
+                break
+            if at + LENGTHS[op] > len(prg):
+                return True
+            if op in LEAVES:
+                break
+            at += LENGTHS[op]
+    return False
+
+
+@pytest.mark.parametrize("tail,open_end", [
+    ([0xEA] * 9, False),                                                     # NOPs end at $FFFF
+    ([0xEA] * 8 + [0xAD], True),                                             # LDA abs at $FFFF
+    ([0xAD, 0x02, 0x03] + [0xEA] * 5 + [0xAD], True),                        # over $FFF7-$FFF9, no opcodes there
+    ([0x8D, 0x02, 0x03] + [0xEA] * 5 + [0xA5], True),
+    ([0x4C, 0x02, 0x03] + [0xEA] * 5 + [0xAD], False),                       # a jump at $FFF7 goes nowhere else
+    ([0x02, 0x02, 0x02] + [0xEA] * 5 + [0xAD], False),                       # nothing falls into the vectors
+    ([0xA5, 0x02, 0x02] + [0xEA] * 5 + [0xAD], False),                       # two bytes end at $FFF8
+])
+def test_images_whose_flow_runs_past_the_end(lib, tail, open_end):
+    """Tails from $FFF7 on, the rest of the image illegal opcodes."""
+    prg = bytes([0x02] * (32768 - len(tail)) + tail)
+    assert runs_past_the_end(prg) == open_end
+    assert bool(lib.t_closed_end(prg, len(prg))) == (not open_end)
+
+
+def test_random_images_agree_with_a_walk_of_the_flow(lib):
+    """Random tails, of all bytes and of few illegal ones, both image sizes."""
+    rng = np.random.default_rng(5)
+    legal = np.array([op for op in range(256) if LENGTHS[op] and op not in LEAVES], dtype=np.uint8)
+    seen = {True: 0, False: 0}
+    for k in range(4000):
+        size = 16384 if k % 2 else 32768
+        tail = rng.integers(0, 256, 32).astype(np.uint8)
+        mostly = rng.random(32) < (0.0, 0.5, 0.9)[k % 3]
+        tail[mostly] = rng.choice(legal, int(mostly.sum()))
+        prg = bytes(size - 32) + bytes(tail)
+        want = runs_past_the_end(prg)
+        seen[want] += 1
+        assert bool(lib.t_closed_end(prg, size)) == (not want), tail.tobytes().hex()
+    assert min(seen.values()) > 200
