@@ -758,8 +758,13 @@ __device__ __forceinline__ std::uint32_t wave_run(WaveCpu& c, std::uint32_t ram,
   s_sub_u32 s[rExit], s[rJ], 0x10000
   UNPACK
   s_and_b32 s[rT], s[rTab], 0xFFFF
+.if SOLO
+  s_cbranch_scc1 .Lw%=_unfit
+  s_cmp_eq_u32 s[rTab], 0   ; the exit table would lie in the 4 GB below
+.endif
   s_cbranch_scc0 .Lw%=_start
-  PACK                      ; a table that is not aligned: nothing runs here
+.Lw%=_unfit:
+  PACK                      ; a table that jumps do not reach: nothing runs here
   s_mov_b32 s[rK], 0
   s_mov_b32 s[rU], %0
   s_mov_b64 exec, -1

@@ -1,5 +1,6 @@
-"""Which kernel steps a batch (nesle_amd/csrc/nes_choice.h), compiled alone and
-without a GPU: the test for images whose flow runs past $FFFF."""
+"""The one-console-per-wave step kernels without a GPU: the rules that choose a
+batch's kernel (nesle_amd/csrc/nes_choice.h, compiled alone) -- images whose
+flow runs past $FFFF -- and where their dispatch tables may lie."""
 
 from __future__ import annotations
 
@@ -90,3 +91,66 @@ def test_random_images_agree_with_a_walk_of_the_flow(lib):
         seen[want] += 1
         assert bool(lib.t_closed_end(prg, size)) == (not want), tail.tobytes().hex()
     assert min(seen.values()) > 200
+
+
+WAVE = build.CSRC / "nes_wave.h"
+
+
+def enter(table: int, solo: bool) -> dict | None:
+    """The assembly's own test of where its dispatch table lies, followed line
+    by line for a table at that address: the registers with which the block is
+    entered, or None where nothing runs in it."""
+    text = WAVE.read_text()
+    at = text.index("  s_mov_b32 s[rTab], s[rJ]")
+    lines = [ln.split(";")[0].strip() for ln in text[at:text.index(".Lw%=_end:", at)].splitlines()]
+    reg = {"rJ": table & 0xFFFFFFFF}
+    scc, skip, k = 0, False, 0
+
+    def value(x: str) -> int:
+        return reg[x[2:-1]] if x.startswith("s[") else int(x, 0)
+
+    while True:
+        op, _, rest = lines[k].partition(" ")
+        a = [x.strip() for x in rest.split(",")]
+        k += 1
+        if op == ".if":
+            assert a == ["SOLO"]
+            skip = not solo
+        elif op == ".endif":
+            skip = False
+        elif skip or not op or op == "UNPACK" or (op.endswith(":") and op != ".Lw%=_start:"):
+            continue
+        elif op == "PACK":
+            return None
+        elif op == ".Lw%=_start:":
+            return reg
+        elif op == "s_mov_b32":
+            reg[a[0][2:-1]] = value(a[1])
+        elif op == "s_sub_u32":
+            reg[a[0][2:-1]] = (value(a[1]) - value(a[2])) & 0xFFFFFFFF
+        elif op == "s_and_b32":
+            reg[a[0][2:-1]] = value(a[1]) & value(a[2])
+            scc = int(reg[a[0][2:-1]] != 0)
+        elif op == "s_cmp_eq_u32":
+            scc = int(value(a[0]) == value(a[1]))
+        elif op in ("s_cbranch_scc0", "s_cbranch_scc1"):
+            if scc == int(op[-1]):
+                k = lines.index(a[0] + ":")
+        else:
+            raise AssertionError(f"unexpected line: {lines[k - 1]}")
+
+
+@pytest.mark.parametrize("solo", [True, False])
+@pytest.mark.parametrize("table", [0x7F0012340000, 0x7F0000010000, 0x7F00FFFF0000, 0x7F0000000000, 0x7F0012340100,
+                                   0x7F0000000100])
+def test_dispatch_tables_are_reached_by_their_low_half(table, solo):
+    """A jump replaces only the low 32 bits of the table's address, so the
+    solo form's exit table (64 KB below) must share its high ones; and the
+    table must be aligned to its 64 KB.  Elsewhere nothing runs in the block."""
+    reg = enter(table, solo)
+    fits = table % 0x10000 == 0 and (not solo or (table - 0x10000) >> 32 == table >> 32)
+    assert (reg is not None) == fits
+    if reg is not None:
+        assert reg["rTab"] == reg["rQ"] == table & 0xFFFFFFFF
+        if solo:
+            assert (table >> 32 << 32 | reg["rExit"]) == table - 0x10000
