@@ -184,6 +184,13 @@ int nesle_set_actions(nesle_batch* b, const void* actions, int dtype, int on_dev
  * step_device/step_stats/step_profile sequences (cuda_module.cu:594-818). */
 int nesle_step(nesle_batch* b, int auto_reset, int stats_mode);
 
+/* Steps so far in which the library chose between its two step kernels
+ * (stats_mode 0, no binding budget, up to 32,768 consoles): how many ran with
+ * one console per wave and how many in lanes, as programs that keep leaving
+ * the former's fast path do.  Counted on the device, so replays of a captured
+ * step count too.  Waits for the batch's stream.  No reference counterpart. */
+int nesle_step_choices(nesle_batch* b, uint64_t* per_wave, uint64_t* lanes);
+
 /* Device view of one buffer (NESLE_VIEW_*, not OAM).  Replaces
  * ram_device/rewards_device/last_done_device (cuda_module.cu:854-902) and
  * frames_device (cuda_module.cu:871-886).  A frame view exists once

@@ -138,6 +138,7 @@ def lib():
         "nesle_reset_envs": (ctypes.c_int, [vp, vp, ctypes.c_int]),
         "nesle_set_actions": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int]),
         "nesle_step": (ctypes.c_int, [vp, ctypes.c_int, ctypes.c_int]),
+        "nesle_step_choices": (ctypes.c_int, [vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]),
         "nesle_get_view": (ctypes.c_int, [vp, ctypes.c_int, ctypes.POINTER(View)]),
         "nesle_copy_to_host": (ctypes.c_int, [vp, ctypes.c_int, vp, ctypes.c_size_t]),
         "nesle_copy_views": (ctypes.c_int, [vp, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(vp),
@@ -263,6 +264,13 @@ class Batch:
 
     def step(self, auto_reset: bool = False, stats_mode: int = 0) -> None:
         _check(lib().nesle_step(self.h, int(auto_reset), stats_mode))
+
+    def step_choices(self) -> tuple[int, int]:
+        """(steps with one console per wave, steps in lanes) of those in which
+        the library chose the kernel."""
+        per_wave, lanes = ctypes.c_uint64(), ctypes.c_uint64()
+        _check(lib().nesle_step_choices(self.h, ctypes.byref(per_wave), ctypes.byref(lanes)))
+        return per_wave.value, lanes.value
 
     def synthetic_step(self, apply_actions: bool = True, auto_reset: bool = False) -> None:
         _check(lib().nesle_synthetic_step(self.h, int(apply_actions), int(auto_reset)))

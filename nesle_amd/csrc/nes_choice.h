@@ -1,11 +1,17 @@
-// nes_choice.h -- which kernel steps a batch: rules without device code of
-// their own, shared by the host library and compiled alone by the CPU tests.
+// nes_choice.h -- which kernel steps a batch: plain rules shared by the host
+// library and the step kernels, compiled alone by the CPU tests.
 #pragma once
 
 #include <cstddef>
 #include <cstdint>
 
 #include "nes_micro.h"
+
+#ifdef __HIPCC__
+#define NESLE_BOTH_SIDES __host__ __device__
+#else
+#define NESLE_BOTH_SIDES
+#endif
 
 namespace nesle {
 
@@ -32,6 +38,56 @@ inline bool closed_end(const std::uint8_t* prg, std::size_t size) {
         if (!leaves && next < kTail) reached[next] = true;
     }
     return true;
+}
+
+// The choice between the one-console-per-wave kernels and the lane kernel, in
+// device memory.  A program the first gain on seldom leaves their assembly
+// for the general path (NMI entry, DMA, PPU control: about a dozen times a
+// frame); one that runs from RAM or polls other registers all the time goes to
+// the lane kernel for a while and is then tried again.
+//
+// A step launches both kernels and the one that is not chosen returns at once:
+// the per-wave kernel reads `next` and leaves it in `now` for the lane kernel
+// behind it, which counts the step (choice_update).  So each step's choice
+// follows from the steps before it on the stream, whether they were enqueued
+// long before any of them ran or are replayed from a captured graph.  Only the
+// kernel depends on it, not the results.  The launch that returns at once costs
+// 3 us of the vector environment's 711 with one console, 9 of 3,517 at 30,001
+// consoles.
+constexpr std::uint32_t kGeneralSlots = 16;
+struct StepChoice {
+    std::uint64_t steps[2];             // taken by [0] one console per wave, [1] the lane kernel
+    std::uint32_t next, now;            // kernel of the next step, of this one
+    std::uint32_t left;                 // steps the lane kernel still takes
+    std::uint32_t over[kGeneralSlots];  // whether the first consoles took the general path too often
+};
+constexpr std::uint32_t kLaneSteps = 64;
+
+// After the step whose kernel is `now`: the next one's.
+NESLE_BOTH_SIDES inline void choice_update(StepChoice& c) {
+    ++c.steps[c.now];
+    if (c.now == 0) {
+        std::uint32_t over = 0;
+        for (std::uint32_t i = 0; i < kGeneralSlots; ++i) over |= c.over[i];
+        if (over == 0) return;
+        c.next = 1;
+        c.left = kLaneSteps;
+    } else if (--c.left == 0) {
+        c.next = 0;
+    }
+}
+
+// Trips through the general path per frame from which on the lane kernel is
+// quicker on a batch of n consoles.  Per 1,024 consoles (one wave per SIMD) a
+// trip costs about 1,100 cycles of 2.4 GHz, and a step of four frames 0.42 ms,
+// at least 2.5 in all, against the lane kernel's 14 (up to 8,192 consoles) or
+// 17 ms: at 4,096 consoles 1,254 trips a frame, 8,192 580, 16,384 280,
+// 32,768 48.
+inline std::uint32_t general_limit(std::uint32_t n) {
+    const double waves = n > 1024 ? n / 1024.0 : 1.0;
+    const double lane_ms = n <= 8192 ? 14.0 : 17.0, wave_ms = 0.42 * waves > 2.5 ? 0.42 * waves : 2.5;
+    const double limit = (lane_ms - wave_ms) * 0.25e-3 * 2.4e9 * 0.8 / ((waves > 2.0 ? waves : 2.0) * 1100.0);
+    return limit > 0.0 ? static_cast<std::uint32_t>(limit) : 0u;
 }
 
 }  // namespace nesle

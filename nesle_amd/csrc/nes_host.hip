@@ -244,11 +244,8 @@ struct nesle_batch {
     double timed_ms = 0.0;        // step kernel
     double timed_reset_ms = 0.0;  // restore kernel of the auto-reset
     std::uint64_t timed_launches = 0;
-    // The choice between the step kernels (wave_pays).
-    static constexpr std::uint32_t kLaneSteps = 64, kOnTrial = 0xFFFFFFFFu;
+    // The choice between the step kernels (nes_choice.h).
     bool closed_end = false;
-    std::uint32_t lane_steps = 0;
-    std::uint32_t* general = nullptr;   // host memory, written by the kernels
     // Pinned host memory that kernels read and write: the actions of a step on
     // their way in, small views on their way out.  A copy between pageable
     // memory and the device waits for the stream, and costs 25-45 us of its
@@ -280,7 +277,6 @@ struct nesle_batch {
         (void)hipFree(d_live_records);
         (void)hipFree(d_step_counts);
         (void)hipFree(d_render_tables);
-        (void)hipHostFree(general);
         (void)hipHostFree(stage_in);
     }
 
@@ -322,6 +318,7 @@ struct nesle_batch {
         add(&d_mask, n);
         add(&d_blob, blob::kBytes);
         add(&d_levels, n);
+        add(&ds.choice, sizeof(nesle::StepChoice));   // all zero: one console per wave
         std::size_t total = 0;
         for (const auto& s : slots) total = align_up(total, 256) + s.bytes;
         hip_check(hipMalloc(&arena, total), "hipMalloc state arena");
@@ -358,41 +355,6 @@ struct nesle_batch {
         ds.prof_opcodes = reinterpret_cast<unsigned long long*>(base + a + b + c);
         ds.prof_pcs = ds.prof_opcodes + 256;
         ds.census = ds.prof_pcs + 65536;
-    }
-
-    // Whether the one-console-per-wave kernels take the next step.  They gain
-    // while a program seldom leaves their assembly for the general path (NMI
-    // entry, DMA, PPU control: about a dozen times a frame); one that runs
-    // from RAM or polls other registers all the time goes to the lane kernel,
-    // and is tried again after kLaneSteps steps.  The first consoles of a
-    // launch report their trips per frame in host memory; the report read
-    // here is that of whatever launch has finished, and only the choice of
-    // the kernel depends on it, not the results.
-    //
-    // The bound: per 1,024 consoles (one wave per SIMD) a trip costs about
-    // 1,100 cycles of 2.4 GHz, and a step of four frames 0.42 ms, at least
-    // 2.5 in all, against the lane kernel's 14 (up to 8,192 consoles) or
-    // 17 ms.  At 4,096 consoles 1,330 trips a frame, 8,192 640, 16,384 300,
-    // 32,768 50.
-    bool wave_pays() {
-        if (!closed_end) return false;
-        auto report = [&](std::uint32_t i) { return __atomic_load_n(general + i, __ATOMIC_RELAXED); };
-        if (lane_steps != 0) {
-            if (--lane_steps != 0) return false;
-            // One step on trial: the next ones wait for its report.
-            for (std::uint32_t i = 0; i < nesle::kGeneralSlots; ++i) __atomic_store_n(general + i, 0u, __ATOMIC_RELAXED);
-            __atomic_store_n(general, kOnTrial, __ATOMIC_RELAXED);
-            return true;
-        }
-        if (report(0) == kOnTrial) return false;
-        const double waves = std::max(1.0, n() / 1024.0);
-        const double lane_ms = n() <= 8192 ? 14.0 : 17.0, wave_ms = std::max(2.5, 0.42 * waves);
-        const double limit = (lane_ms - wave_ms) * 0.25e-3 * 2.4e9 * 0.8 / (std::max(2.0, waves) * 1100.0);
-        std::uint32_t most = 0;
-        for (std::uint32_t i = 0; i < nesle::kGeneralSlots; ++i) most = std::max(most, report(i));
-        if (most <= limit) return true;
-        lane_steps = kLaneSteps;
-        return false;
     }
 
     void refresh_obs() { hip_check(nesle::launch_ram_obs(ds, d_obs, stream), "ram_obs_kernel"); }
@@ -621,14 +583,7 @@ void open_batch(nesle_batch* b, const nesle_config* cfg) {
     s.clip = b->cfg.clip;
     s.time_penalty = b->cfg.time_penalty;
     b->closed_end = nesle::closed_end(b->rom.prg.data(), b->rom.prg.size());
-    void* general = nullptr;
-    hip_check(hipHostMalloc(&general, sizeof(std::uint32_t) * nesle::kGeneralSlots, hipHostMallocMapped),
-              "hipHostMalloc general-path reports");
-    std::memset(general, 0, sizeof(std::uint32_t) * nesle::kGeneralSlots);
-    b->general = static_cast<std::uint32_t*>(general);
-    void* seen = nullptr;
-    hip_check(hipHostGetDevicePointer(&seen, general, 0), "hipHostGetDevicePointer");
-    s.general = static_cast<std::uint32_t*>(seen);
+    s.general_limit = nesle::general_limit(s.n);
     b->allocate();
     b->host_to_device(b->d_prg, b->rom.prg.data(), b->rom.prg.size(), "upload PRG ROM");
     if (!b->rom.chr.empty()) b->host_to_device(b->d_chr, b->rom.chr.data(), b->rom.chr.size(), "upload CHR ROM");
@@ -837,7 +792,7 @@ int nesle_step(nesle_batch* b, int auto_reset, int stats_mode) {
             s.prof_pcs = nullptr;
         }
         if (stats_mode != 3) s.census = nullptr;
-        s.per_wave = stats_mode == 0 && b->wave_pays() ? 1u : 0u;
+        if (!b->closed_end) s.choice = nullptr;
         nesle_batch::Marks ev{};
         if (b->timing) {
             b->fold_events(false);
@@ -1084,6 +1039,19 @@ int nesle_set_stream(nesle_batch* b, void* hip_stream) {
         if (b == nullptr) throw InvalidArgument("null batch");
         b->sync();
         b->stream = static_cast<hipStream_t>(hip_stream);
+    });
+}
+
+int nesle_step_choices(nesle_batch* b, std::uint64_t* per_wave, std::uint64_t* lanes) {
+    return guarded([&] {
+        if (b == nullptr || per_wave == nullptr || lanes == nullptr) throw InvalidArgument("null argument");
+        b->activate();
+        std::uint64_t steps[2] = {};
+        static_assert(offsetof(nesle::StepChoice, steps) == 0, "copied from there");
+        hip_check(hipMemcpyAsync(steps, b->ds.choice, sizeof(steps), hipMemcpyDeviceToHost, b->stream), "copy step choices");
+        b->sync();
+        *per_wave = steps[0];
+        *lanes = steps[1];
     });
 }
 

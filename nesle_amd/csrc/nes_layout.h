@@ -58,6 +58,8 @@ enum RewardKind : std::uint32_t {
     kRewardXDelta = 1,  // clip(int16(x - x_prev), -clip, clip) - time_penalty; done = RAM[done_addr] == 0
 };
 
+struct StepChoice;   // nes_choice.h
+
 struct DeviceState {
     std::uint32_t n;           // consoles
     std::uint32_t pitch;       // interleave pitch (multiple of 256, >= n)
@@ -140,13 +142,11 @@ struct DeviceState {
     std::uint8_t* lat_sy;      // [n]
     std::uint8_t* lat_ctrl;    // [n]
 
-    // The one-console-per-wave kernels may run this step (nes_host.hip says
-    // when), and where they report how often their general path was taken:
-    // kGeneralSlots words of host memory.
-    std::uint32_t per_wave;
-    std::uint32_t* general;
+    // The choice between the step kernels (nes_choice.h), or null: the lane
+    // kernel.  And the trips through the general path per frame it turns on.
+    StepChoice* choice;
+    std::uint32_t general_limit;
 };
-constexpr std::uint32_t kGeneralSlots = 16;
 
 // Step-kernel census (stats mode 3): what the waves of one launch did, summed
 // over waves.  A "wave-iteration" is one trip of the step loop (one emulated

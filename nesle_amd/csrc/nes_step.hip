@@ -57,6 +57,7 @@
 
 #include "nes_device.h"
 #include "nes_launch.h"
+#include "nes_choice.h"
 #include "nes_layout.h"
 #include "nes_micro.h"
 
@@ -630,6 +631,15 @@ struct WaveCensus {
     }
 };
 
+#if NESLE_STEP_PART == 1 || NESLE_STEP_PART == 2
+// Behind a one-console-per-wave kernel: whether that one has taken the step.
+__device__ __forceinline__ bool taken_per_wave(StepChoice* c) {
+    const bool taken = c->now == 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) choice_update(*c);
+    return taken;
+}
+#endif
+
 // ---- the step kernel ---------------------------------------------------------------
 // kStats: 0 none, 1 per-console counters, 2 counters + opcode/PC histograms,
 // 3 counters + the census of the launch (WaveCensus).
@@ -648,6 +658,11 @@ __global__ void __launch_bounds__(kFull ? 256 : kMaxBlock) step_kernel(DeviceSta
     const std::uint32_t slot = wave * L + lane;
     const std::uint32_t env = xcd_block(blockIdx.x, gridDim.x) * ((T >> 6) * L) + slot;
     const bool mine = lane < L && env < s.n;
+#if NESLE_STEP_PART == 1 || NESLE_STEP_PART == 2
+    if constexpr (kStats == 0 && !kBudget) {
+        if (s.choice != nullptr && taken_per_wave(s.choice)) return;
+    }
+#endif
 
     {   // PRG ROM (a 16 KB image mirrored to 32 KB) and the microcode table.
         const std::uint32_t words = (s.prg_mask + 1) / 16;
@@ -1513,16 +1528,21 @@ hipError_t launch_step_narrow(const DeviceState& s, std::uint32_t waves, std::ui
     return launch_layout<false>(s, g, frameskip, max_instr, stats_mode, stream);
 }
 #elif NESLE_STEP_PART == 0
-hipError_t launch_step(const DeviceState& s, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
+hipError_t launch_step(const DeviceState& state, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
                        hipStream_t stream) {
+    DeviceState s = state;
+    if (stats_mode != 0 || budget_binds(max_instr) || s.n > kWaveMaxConsoles) s.choice = nullptr;
     // One console per wave up to 32,768 consoles: there the wave kernel takes
     // 13.2 ms on a program that never idles and 4.75 on one that waits in
     // JMP *, this file's 17.3 and 5.98; at 40,960 16.7 and about 6 against
     // 18.6 and 6.03.  Its solo form up to 4,096, four waves per SIMD: 2.74 ms
     // there against 2.81, 2.46 against 2.80 at 1,000; at 8,192 3.92 against
     // 3.43.
-    if (stats_mode == 0 && !budget_binds(max_instr) && s.per_wave != 0 && s.n <= kWaveMaxConsoles)
-        return s.n <= kSoloMaxConsoles ? launch_step_solo(s, frameskip, stream) : launch_step_wave(s, frameskip, stream);
+    if (s.choice != nullptr) {   // the kernel that is not chosen returns at once (nes_choice.h)
+        const hipError_t e = s.n <= kSoloMaxConsoles ? launch_step_solo(s, frameskip, stream)
+                                                     : launch_step_wave(s, frameskip, stream);
+        if (e != hipSuccess) return e;
+    }
     const std::uint32_t waves = waves_per_group();
     const Geometry g = geometry(s.n, waves);
     if (g.full) return launch_step_full(s, frameskip, max_instr, stats_mode, stream);

@@ -24,7 +24,7 @@
 //
 // Statistics and binding instruction budgets stay with the lane kernel, as do
 // images whose flow can run past their end, and programs that take the general
-// path too often (nes_host.hip): an instruction there costs about 1,100
+// path too often (nes_choice.h): an instruction there costs about 1,100
 // cycles of a SIMD, where a lane of the lane kernel shares 1,400 with 63
 // others.
 //
@@ -105,6 +105,10 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
     const std::uint32_t env = env0 + wave;
     const std::uint32_t P = s.pitch;
     const bool mine = env < s.n;
+
+    const bool lanes = s.choice->next != 0;   // the lane kernel behind takes this step
+    if (blockIdx.x == 0 && tid == 0) s.choice->now = lanes ? 1u : 0u;
+    if (lanes) return;
 
     {   // PRG ROM (a 16 KB image mirrored to 32 KB) between its guards.
         const std::uint32_t words = (s.prg_mask + 1) / 16;
@@ -368,9 +372,10 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
         }
         flags = c.flags;
         frames = c.r32(reg::kFrames);
-        // How often the first consoles took the general path, per frame.
-        if (blockIdx.x < kGeneralSlots && wave == 0 && lane == 0 && frameskip != 0)
-            reload(c.s)->general[blockIdx.x] = general / frameskip;
+        if (blockIdx.x < kGeneralSlots && wave == 0 && lane == 0 && frameskip != 0) {
+            KState* k = reload(c.s);
+            k->choice->over[blockIdx.x] = general / frameskip > k->general_limit ? 1u : 0u;
+        }
     }
     __syncthreads();
 

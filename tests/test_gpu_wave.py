@@ -117,29 +117,75 @@ def poll_rom() -> bytes:
     return nrom_bytes(2, code={0x8000: loop, 0x9000: [0x40]}, reset=0x8000, nmi=0x9000, irq=0x9000)
 
 
-@pytest.mark.gpu
-def test_polling_program_moves_to_the_lane_kernel():
-    """After its first steps the batch takes the lane kernel (quicker there);
-    the results stay the oracle's through the change and the trial steps."""
-    n, steps = 8200, 70
+def polled(b: abi.Batch, run, steps: int, pads: np.ndarray) -> None:
+    """`steps` frame-skip-1 steps of poll_rom through `run`, all enqueued
+    before any is waited for; sampled consoles end as the oracle's."""
     rom = poll_rom()
-    b, cons = abi.Batch(rom, n, frameskip=1), {e: O.Oracle(rom) for e in (0, 4100, n - 1)}
-    for c in cons.values():
+    sample = (0, b.n // 2, b.n - 1)
+    for _ in range(steps):
+        run()
+    for e in sample:
+        c = O.Oracle(rom)
         c.set_reward()
-    b.set_timing(True)
-    took = []
-    for k in range(steps):
-        m = masks_for(8, n, k)
-        b.set_actions(m)
-        b.step()
-        before = sum(took)
-        took.append(b.timing()[0] - before)     # synchronises: the report is in
-        for e, c in cons.items():
-            c.step(int(m[e]), 1)
-    for e, c in cons.items():
+        for _ in range(steps):
+            c.step(int(pads[e]), 1)
         got, want = b.save_state(e), c.save()
         assert np.array_equal(got, want), f"console {e}: {first_diff(got, want)}"
-    assert max(took[2:60]) < 0.5 * took[0], took
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [60, 8200])
+def test_polling_program_moves_to_the_lane_kernel(n):
+    """The first step runs with one console per wave and reports; the lane
+    kernel takes the next 64, then one is tried again.  Nothing here waits
+    between the steps."""
+    say(f"[gpu] kernel choice: polling program N={n}")
+    b, pads = abi.Batch(poll_rom(), n, frameskip=1), masks_for(8, n, 0)
+    b.set_actions(pads)
+    polled(b, b.step, 70, pads)
+    assert b.step_choices() == (2, 68)
+
+
+@pytest.mark.gpu
+def test_captured_steps_choose_when_they_run():
+    """A step captured before any has run: the replays of its graph move to the
+    lane kernel as eager steps do, and the eager steps between them count."""
+    import torch
+
+    n = 60
+    say(f"[gpu] kernel choice: captured step N={n}")
+    b, pads = abi.Batch(poll_rom(), n, frameskip=1), masks_for(8, n, 0)
+    stream = torch.cuda.Stream()
+    b.set_stream(stream.cuda_stream)
+    b.set_actions(pads)
+    b.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        b.step()
+    assert b.step_choices() == (0, 0)
+    turn = iter(range(1000))
+
+    def run():
+        if next(turn) % 3 == 2:
+            b.step()
+        else:
+            with torch.cuda.stream(stream):
+                graph.replay()
+
+    polled(b, run, 70, pads)
+    assert b.step_choices() == (2, 68)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,chooses", [(60, True), (4097, True), (32768, True), (32769, False)])
+def test_ordinary_programs_stay_with_one_console_per_wave(n, chooses):
+    """Above 32,768 consoles, and under statistics, there is no choice."""
+    say(f"[gpu] kernel choice: ordinary program N={n}")
+    b = abi.Batch(synthrom.make_rom(5).rom, n, frameskip=2)
+    for k in range(5):
+        b.set_actions(masks_for(9, n, k))
+        b.step(stats_mode=1 if k == 2 else 0)
+    assert b.step_choices() == ((4, 0) if chooses else (0, 0))
 
 
 def vector_rom(irq: int, flow: list[int]) -> bytes:

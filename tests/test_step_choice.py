@@ -1,6 +1,6 @@
 """The one-console-per-wave step kernels without a GPU: the rules that choose a
 batch's kernel (nesle_amd/csrc/nes_choice.h, compiled alone) -- images whose
-flow runs past $FFFF -- and where their dispatch tables may lie."""
+flow runs past $FFFF, the choice from step to step -- and where their dispatch tables may lie."""
 
 from __future__ import annotations
 
@@ -20,7 +20,22 @@ pytestmark = pytest.mark.skipif(CXX is None, reason="no host C++ compiler")
 SHIM = r"""
 #include "nes_choice.h"
 using namespace nesle;
-extern "C" int t_closed_end(const std::uint8_t* prg, std::size_t size) { return closed_end(prg, size); }
+extern "C" {
+int t_closed_end(const std::uint8_t* prg, std::size_t size) { return closed_end(prg, size); }
+// `steps` steps of a program that goes over the limit in the per-wave steps
+// for which over[step] is set; the kernel of each into out.
+void t_choices(const std::uint8_t* over, std::uint8_t* out, std::uint32_t steps) {
+    StepChoice c{};
+    for (std::uint32_t k = 0; k < steps; ++k) {
+        c.now = c.next;
+        if (c.now == 0)
+            for (std::uint32_t i = 0; i < kGeneralSlots; ++i) c.over[i] = over[k] && i == k % kGeneralSlots;
+        out[k] = static_cast<std::uint8_t>(c.now);
+        choice_update(c);
+    }
+}
+std::uint32_t t_limit(std::uint32_t n) { return general_limit(n); }
+}
 """
 
 
@@ -32,6 +47,7 @@ def lib(tmp_path_factory):
                     str(work / "shim.so")], check=True, capture_output=True, text=True)
     L = ctypes.CDLL(str(work / "shim.so"))
     L.t_closed_end.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+    L.t_choices.argtypes = [ctypes.c_char_p, ctypes.c_char_p, ctypes.c_uint32]
     return L
 
 
@@ -91,6 +107,30 @@ def test_random_images_agree_with_a_walk_of_the_flow(lib):
         seen[want] += 1
         assert bool(lib.t_closed_end(prg, size)) == (not want), tail.tobytes().hex()
     assert min(seen.values()) > 200
+
+
+def kernels(lib, over: list[bool]) -> list[int]:
+    """0 (one console per wave) or 1 (the lane kernel) for each step."""
+    out = ctypes.create_string_buffer(len(over))
+    lib.t_choices(bytes(over), out, len(over))
+    return list(out.raw)
+
+
+def test_kernel_of_each_step(lib):
+    """No step on the general path beyond the first; 64 lane steps follow one."""
+    assert kernels(lib, [False] * 200) == [0] * 200
+    always = kernels(lib, [True] * 140)
+    assert always[:66] == [0] + [1] * 64 + [0]
+    # One bad step among good ones, wherever it falls.
+    for at in (0, 1, 17):
+        over = [k == at for k in range(at + 70)]
+        assert kernels(lib, over) == [0] * (at + 1) + [1] * 64 + [0] * 5
+
+
+def test_limit_falls_as_the_batch_grows(lib):
+    assert [lib.t_limit(n) for n in (4096, 8192, 16384, 32768)] == [1254, 580, 280, 48]
+    limits = [lib.t_limit(n) for n in range(1, 32769)]
+    assert min(limits) == 48 and max(limits) < 3000
 
 
 WAVE = build.CSRC / "nes_wave.h"
