@@ -44,7 +44,10 @@ inline bool closed_end(const std::uint8_t* prg, std::size_t size) {
 // device memory.  A program the first gain on seldom leaves their assembly
 // for the general path (NMI entry, DMA, PPU control: about a dozen times a
 // frame); one that runs from RAM or polls other registers all the time goes to
-// the lane kernel for a while and is then tried again.
+// the lane kernel for a while and is then tried again, for one step at first: a
+// step wholly on the general path takes some 430 ms at 32,768 consoles, against
+// the lane kernel's 17, so the while grows from 64 steps by fours to 4,096
+// (0.6 % of them) and is 64 again once a run of steps as long as it went well.
 //
 // A step launches both kernels and the one that is not chosen returns at once:
 // the per-wave kernel reads `next` and leaves it in `now` for the lane kernel
@@ -59,9 +62,10 @@ struct StepChoice {
     std::uint64_t steps[2];             // taken by [0] one console per wave, [1] the lane kernel
     std::uint32_t next, now;            // kernel of the next step, of this one
     std::uint32_t left;                 // steps the lane kernel still takes
+    std::uint32_t level, good;          // its next stay, kLaneSteps << 2 level; good steps since the last one
     std::uint32_t over[kGeneralSlots];  // whether the first consoles took the general path too often
 };
-constexpr std::uint32_t kLaneSteps = 64;
+constexpr std::uint32_t kLaneSteps = 64, kMaxLevel = 3;
 
 // After the step whose kernel is `now`: the next one's.
 NESLE_BOTH_SIDES inline void choice_update(StepChoice& c) {
@@ -69,9 +73,15 @@ NESLE_BOTH_SIDES inline void choice_update(StepChoice& c) {
     if (c.now == 0) {
         std::uint32_t over = 0;
         for (std::uint32_t i = 0; i < kGeneralSlots; ++i) over |= c.over[i];
-        if (over == 0) return;
+        const std::uint32_t stay = kLaneSteps << 2 * c.level;
+        if (over == 0) {
+            if (c.level != 0 && ++c.good >= stay) c.level = c.good = 0;
+            return;
+        }
         c.next = 1;
-        c.left = kLaneSteps;
+        c.left = stay;
+        c.good = 0;
+        if (c.level < kMaxLevel) ++c.level;
     } else if (--c.left == 0) {
         c.next = 0;
     }

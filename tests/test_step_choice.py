@@ -117,14 +117,34 @@ def kernels(lib, over: list[bool]) -> list[int]:
 
 
 def test_kernel_of_each_step(lib):
-    """No step on the general path beyond the first; 64 lane steps follow one."""
+    """Steps within the limit stay; a step over it is followed by 64 lane steps."""
     assert kernels(lib, [False] * 200) == [0] * 200
-    always = kernels(lib, [True] * 140)
-    assert always[:66] == [0] + [1] * 64 + [0]
     # One bad step among good ones, wherever it falls.
     for at in (0, 1, 17):
         over = [k == at for k in range(at + 70)]
         assert kernels(lib, over) == [0] * (at + 1) + [1] * 64 + [0] * 5
+
+
+def test_trials_of_a_program_that_stays_over_the_limit_grow_rare(lib):
+    """One step is tried after 64, 256, 1,024 and from then on 4,096 lane steps."""
+    got = kernels(lib, [True] * 20000)
+    tried = [k for k, kernel in enumerate(got) if kernel == 0]
+    assert tried[:4] == [0, 65, 322, 1347]
+    assert set(np.diff(tried[3:])) == {4097}
+    # At 32,768 consoles a trial takes some 430 ms, a lane step 17: under 1 %.
+    assert (len(tried) - 4) * 430 < 0.01 * (20000 - 1347) * 17
+
+
+def test_trials_start_over_after_a_run_of_good_steps(lib):
+    """Twice over the limit in a row: the stays are 64 and 256; the third one
+    is 64 again only after 1,024 good steps, the length it would have had."""
+    for good, third in ((1023, 1024), (1024, 64)):
+        first = 1 + 64 + 1 + 256            # both bad steps and their stays
+        over = [k in (0, 65, first + good) for k in range(first + good + 1200)]
+        got = kernels(lib, over)
+        assert got[:first + good + 1] == [0] + [1] * 64 + [0] + [1] * 256 + [0] * (good + 1)
+        rest = got[first + good + 1:]
+        assert rest[:third] == [1] * third and rest[third] == 0
 
 
 def test_limit_falls_as_the_batch_grows(lib):
