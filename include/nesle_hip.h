@@ -184,6 +184,12 @@ int nesle_set_actions(nesle_batch* b, const void* actions, int dtype, int on_dev
  * step_device/step_stats/step_profile sequences (cuda_module.cu:594-818). */
 int nesle_step(nesle_batch* b, int auto_reset, int stats_mode);
 
+/* only != 0: every later step of this batch takes the step kernel that runs
+ * consoles in lanes, whatever the batch's size and program (results are the
+ * same; for comparing the kernels).  0: the library chooses, as it does by
+ * default.  No reference counterpart. */
+int nesle_set_lane_kernel(nesle_batch* b, int only);
+
 /* Steps so far in which the library chose between its two step kernels
  * (stats_mode 0, no binding budget, up to 32,768 consoles): how many ran with
  * one console per wave and how many in lanes, as programs that keep leaving

@@ -138,6 +138,7 @@ def lib():
         "nesle_reset_envs": (ctypes.c_int, [vp, vp, ctypes.c_int]),
         "nesle_set_actions": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int]),
         "nesle_step": (ctypes.c_int, [vp, ctypes.c_int, ctypes.c_int]),
+        "nesle_set_lane_kernel": (ctypes.c_int, [vp, ctypes.c_int]),
         "nesle_step_choices": (ctypes.c_int, [vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]),
         "nesle_get_view": (ctypes.c_int, [vp, ctypes.c_int, ctypes.POINTER(View)]),
         "nesle_copy_to_host": (ctypes.c_int, [vp, ctypes.c_int, vp, ctypes.c_size_t]),
@@ -264,6 +265,11 @@ class Batch:
 
     def step(self, auto_reset: bool = False, stats_mode: int = 0) -> None:
         _check(lib().nesle_step(self.h, int(auto_reset), stats_mode))
+
+    def set_lane_kernel(self, only: bool) -> None:
+        """True: every later step takes the kernel that runs consoles in lanes;
+        False: the library chooses."""
+        _check(lib().nesle_set_lane_kernel(self.h, int(only)))
 
     def step_choices(self) -> tuple[int, int]:
         """(steps with one console per wave, steps in lanes) of those in which

@@ -245,7 +245,7 @@ struct nesle_batch {
     double timed_reset_ms = 0.0;  // restore kernel of the auto-reset
     std::uint64_t timed_launches = 0;
     // The choice between the step kernels (nes_choice.h).
-    bool closed_end = false;
+    bool closed_end = false, lanes_only = false;
     // Pinned host memory that kernels read and write: the actions of a step on
     // their way in, small views on their way out.  A copy between pageable
     // memory and the device waits for the stream, and costs 25-45 us of its
@@ -792,7 +792,7 @@ int nesle_step(nesle_batch* b, int auto_reset, int stats_mode) {
             s.prof_pcs = nullptr;
         }
         if (stats_mode != 3) s.census = nullptr;
-        if (!b->closed_end) s.choice = nullptr;
+        if (!b->closed_end || b->lanes_only) s.choice = nullptr;
         nesle_batch::Marks ev{};
         if (b->timing) {
             b->fold_events(false);
@@ -1039,6 +1039,13 @@ int nesle_set_stream(nesle_batch* b, void* hip_stream) {
         if (b == nullptr) throw InvalidArgument("null batch");
         b->sync();
         b->stream = static_cast<hipStream_t>(hip_stream);
+    });
+}
+
+int nesle_set_lane_kernel(nesle_batch* b, int only) {
+    return guarded([&] {
+        if (b == nullptr) throw InvalidArgument("null batch");
+        b->lanes_only = only != 0;
     });
 }
 

@@ -73,6 +73,7 @@ def test_frames_at_power_on_and_after_reset():
     _check(b, {e: O.Oracle(rom) for e in range(n)}, "after reset")
 
 
+@pytest.mark.usefixtures("step_kernel")
 @pytest.mark.parametrize("rom_seed,frameskip,steps", [(7, 4, 16), (3, 1, 24), (9, 3, 10)])
 def test_frames_track_oracle_over_steps(rom_seed, frameskip, steps):
     rom = _rom(rom_seed)
@@ -100,6 +101,7 @@ def test_frames_with_instruction_budget():
             _check(b, oracles, f"step {k}")
 
 
+@pytest.mark.usefixtures("step_kernel")
 @pytest.mark.parametrize("variant", ["horizontal", "four_screen", "chr_ram"])
 def test_frames_mirroring_and_chr_ram(variant):
     rom = _rom(5, mirroring=variant if variant != "chr_ram" else "vertical", chr_ram=variant == "chr_ram")
@@ -210,6 +212,7 @@ def test_frames_of_crafted_sprite_layouts():
     _check(b, oracles, "crafted sprites")
 
 
+@pytest.mark.usefixtures("step_kernel")
 @pytest.mark.parametrize("num_envs", [4096])
 def test_frames_full_size_sampled(num_envs):
     rom = _rom(11)
@@ -244,6 +247,7 @@ def test_frames_off_batch_refuses_render():
         abi.Batch(rom, 4, frameskip=4).render(0)
 
 
+@pytest.mark.usefixtures("step_kernel")
 def test_pixel_workload_full_size_sampled():
     """The pixel-observation workload at its full size: 16,384 consoles,
     frame-skip 4, an 84x84 gray frame of every console rendered after every
@@ -272,6 +276,7 @@ def _record_matches(rec: np.ndarray, pres: np.ndarray, tag: str) -> None:
                                   err_msg=f"{tag}: nametables")
 
 
+@pytest.mark.usefixtures("step_kernel")
 def test_status_bar_rom_pixel_workload_full_size_with_auto_resets():
     """The pixel workload on the status-bar ROM (sprite-0 timed mid-frame
     $2005 writes, IRQ-free): 16,384 consoles, frame-skip 4, 4 snapshot levels
@@ -335,6 +340,7 @@ def _h(a: np.ndarray) -> str:
     return f"{O.fnv1a_np(np.ascontiguousarray(a)):016x}"
 
 
+@pytest.mark.usefixtures("step_kernel")
 @pytest.mark.parametrize("rom_seed", [1, 2, 3])
 def test_live_frames_match_the_reference_core_golden(rom_seed):
     """One console over 600 frames (frame-skip 1, the single-env workload):

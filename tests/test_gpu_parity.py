@@ -138,10 +138,11 @@ def test_ragged_batch_sizes_sampled(num_envs):
 
 
 def test_kernel_builds_agree_across_batch_sizes():
-    """The production step kernel (no statistics, no frame budget) comes from
-    three builds with different scheduler flags: all RAM in LDS (up to 8,192
+    """The lane kernel without statistics or frame budget comes from three
+    builds with different scheduler flags: all RAM in LDS (up to 8,192
     consoles), the split layout at 16 or 32 consoles per wave (16,384 and
-    32,768) and at 64 (65,536).  The first 8,192 consoles of each batch, given
+    32,768) and at 64 (65,536); the library chooses only the last by itself,
+    and one console per wave for the smaller batches.  The first 8,192 consoles of each batch, given
     the same pads, end every one of 4 steps with identical rewards and done
     flags, and the last with identical RAM (all 8,192) and canonical state (a
     sample).  The statistics counters, which only statistics steps write,
@@ -152,15 +153,17 @@ def test_kernel_builds_agree_across_batch_sizes():
     masks = [masks_for(777, sizes[-1], k) for k in range(4)]
     sample = [0, 1, 63, 64, 4095, n0 - 1]
     ref = None
-    for n in sizes:
-        say(f"[gpu] kernel builds agree: N={n} fs=4 steps=4")
+    for n, lanes in [(n, True) for n in sizes] + [(8192, False), (32768, False)]:
+        say(f"[gpu] kernel builds agree: N={n} lanes={lanes} fs=4 steps=4")
         b = abi.Batch(rom, n, frameskip=4, reward_kind=abi.REWARD_XDELTA, x_lo=synthrom.X_LO, x_hi=synthrom.X_HI,
                       done_addr=synthrom.DONE_BYTE, clip=15, time_penalty=0.25)
+        b.set_lane_kernel(lanes)
         per_step = []
         for k in range(4):
             b.set_actions(masks[k][:n])
             b.step()
             per_step.append((b.host(abi.VIEW_REWARDS)[:n0].copy(), b.host(abi.VIEW_DONES)[:n0].copy()))
+        assert b.step_choices() == (0 if lanes else 4, 0)
         # Steps without statistics leave the per-console counters as created: zero.
         assert not b.host(abi.VIEW_FRAMES).any() and not b.host(abi.VIEW_INSTRUCTIONS).any()
         got = (per_step, b.host(abi.VIEW_RAM)[:n0].copy(), [b.save_state(e) for e in sample])
@@ -177,6 +180,7 @@ def test_kernel_builds_agree_across_batch_sizes():
             assert np.array_equal(c, a), f"N={n} env {e}: {first_diff(c, a)}"
 
 
+@pytest.mark.usefixtures("step_kernel")
 def test_snapshot_autoreset_xdelta_reward():
     """Config 3 in miniature: 8 snapshots captured after seeded warm-up frames,
     done byte patched so episodes end within the run, x-delta reward with time
@@ -392,6 +396,7 @@ def test_benchmark_workload_soak_full_size_sampled():
     assert ends >= 5 * len(sample)
 
 
+@pytest.mark.usefixtures("step_kernel")
 def test_reset_envs_and_state_roundtrip():
     """Masked reset returns exactly the selected consoles to power-on; a saved
     state loaded into other consoles makes them identical; int64 device
@@ -430,6 +435,7 @@ def test_reset_envs_and_state_roundtrip():
     np.testing.assert_array_equal(b2.host(abi.VIEW_RAM), b3.host(abi.VIEW_RAM))
 
 
+@pytest.mark.usefixtures("step_kernel")
 def test_full_size_snapshot_reset_properties():
     """Size-independent properties at 65,536 consoles with 8 snapshot levels:
     two batches fed the same actions stay identical (RAM of every console);
@@ -535,6 +541,7 @@ def test_profile_step_clears_and_replays_in_a_graph():
             assert np.array_equal(cap.save_state(e), eager.save_state(e)), f"replay {k} env {e}"
 
 
+@pytest.mark.usefixtures("step_kernel")
 @pytest.mark.parametrize("num_envs", [64, 16384])
 def test_nrom128_cold_boot_nmi_loop_and_autoreset(num_envs):
     """A 16 KB PRG image (NROM-128) mirrored at $8000 and $C000 (the

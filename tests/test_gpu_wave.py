@@ -1,7 +1,8 @@
 """The one-console-per-wave step kernels (nes_step_wave.hip, nes_step_solo.hip),
-which run plain steps of up to 32,768 consoles.  A statistics step runs the
-lane kernel, which the oracle tests pin, so twin batches stepped with and
-without statistics must agree in every byte: over programs that take each
+which run plain steps of up to 32,768 consoles, and the choice between them and
+the lane kernel.  A statistics step runs the lane kernel, which the oracle
+tests pin, so three batches -- stepped by these kernels, by the lane kernel
+without statistics and by it with them -- must agree in every byte: over programs that take each
 side path (I/O, PRG RAM, code in RAM, stack and address wraps, illegal
 opcodes, OAM DMA from every kind of page, the idle loop) and over sizes at the
 edges of the workgroup shapes.  Programs that run into and over the vectors
@@ -62,23 +63,29 @@ ROMS = {
 }
 
 
-def twins(rom: bytes, n: int, frameskip: int, steps: int, seed: int) -> None:
-    a, b = abi.Batch(rom, n, frameskip=frameskip), abi.Batch(rom, n, frameskip=frameskip)
+def agree(rom: bytes, n: int, frameskip: int, steps: int, seed: int) -> None:
+    a, lanes, b = (abi.Batch(rom, n, frameskip=frameskip) for _ in range(3))
+    lanes.set_lane_kernel(True)
     sample = sorted({0, 1 % n, n // 2, n - 1, *np.random.default_rng(n).integers(0, n, 12).tolist()})
     for k in range(steps):
         m = masks_for(seed, n, k)
-        for batch, stats in ((a, 0), (b, 1)):
+        for batch, stats in ((a, 0), (lanes, 0), (b, 1)):
             batch.set_actions(m)
             batch.step(auto_reset=k % 3 == 1, stats_mode=stats)
         for view in (abi.VIEW_REWARDS, abi.VIEW_DONES, abi.VIEW_RAM):
-            assert np.array_equal(a.host(view), b.host(view)), f"step {k} view {view}"
+            want = b.host(view)
+            assert np.array_equal(a.host(view), want), f"step {k} view {view}"
+            assert np.array_equal(lanes.host(view), want), f"step {k} view {view}, lane kernel"
+    assert a.step_choices()[0] >= 1 and lanes.step_choices() == (0, 0)
     # A console stopped by an illegal opcode in the middle of a step keeps the
     # step's earlier vblank only under statistics (which capture every one).
+    assert np.array_equal(a.host(abi.VIEW_PRESENT), lanes.host(abi.VIEW_PRESENT))
     for e in np.flatnonzero((a.host(abi.VIEW_PRESENT) != b.host(abi.VIEW_PRESENT)).any(axis=1)):
         assert a.save_state(int(e))[O.OFF["fault"]] & 1, f"presentation record of console {e}"
     for e in sample:
-        got, want = a.save_state(e), b.save_state(e)
-        assert np.array_equal(got, want), f"console {e}: {first_diff(got, want)}"
+        want = b.save_state(e)
+        for got in (a.save_state(e), lanes.save_state(e)):
+            assert np.array_equal(got, want), f"console {e}: {first_diff(got, want)}"
 
 
 @pytest.mark.gpu
@@ -87,7 +94,7 @@ def twins(rom: bytes, n: int, frameskip: int, steps: int, seed: int) -> None:
 def test_programs_agree_with_the_lane_kernel(name, n):
     """60 consoles: the solo form; 4,160: two workgroups on some CUs."""
     say(f"[gpu] wave kernel: {name} N={n}")
-    twins(ROMS[name](), n, 4, 9, 31)
+    agree(ROMS[name](), n, 4, 9, 31)
 
 
 @pytest.mark.gpu
@@ -98,7 +105,7 @@ def test_sizes_agree_with_the_lane_kernel(n, frameskip):
     consoles in workgroups of 12 end past the row pitch of 2,816), the ends of
     both forms' ranges."""
     say(f"[gpu] wave kernel: N={n} fs={frameskip}")
-    twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 77)
+    agree(synthrom.make_rom(2026).rom, n, frameskip, 4, 77)
 
 
 @pytest.mark.gpu
@@ -107,7 +114,7 @@ def test_workgroups_of_twelve_waves_agree_with_the_lane_kernel(n, frameskip):
     """Both sides of the sizes that take 12 waves per workgroup instead of 16,
     ragged: one, one and a half and three rounds of workgroups on the chip."""
     say(f"[gpu] wave kernel, 12 or 16 waves: N={n} fs={frameskip}")
-    twins(synthrom.make_rom(2026).rom, n, frameskip, 4, 78)
+    agree(synthrom.make_rom(2026).rom, n, frameskip, 4, 78)
 
 
 def poll_rom() -> bytes:
