@@ -1483,12 +1483,13 @@ hipError_t launch_layout(const DeviceState& s, const Geometry& g, std::uint32_t 
 
 #endif
 #if NESLE_STEP_PART == 0
-// Waves per workgroup: NESLE_WAVES_PER_GROUP (4, 8 or 16) overrides the default.
-std::uint32_t waves_per_group() {
+// Waves per workgroup of the lane kernel: NESLE_WAVES_PER_GROUP (4, 8 or 16)
+// overrides the default, and asks for that kernel; 0 where it does not.
+std::uint32_t asked_waves_per_group() {
     static const std::uint32_t w = [] {
         const char* e = std::getenv("NESLE_WAVES_PER_GROUP");
         const long v = e != nullptr ? std::strtol(e, nullptr, 10) : 0;
-        return (v == 4 || v == 8 || v == 16) ? static_cast<std::uint32_t>(v) : 4u;
+        return (v == 4 || v == 8 || v == 16) ? static_cast<std::uint32_t>(v) : 0u;
     }();
     return w;
 }
@@ -1531,7 +1532,8 @@ hipError_t launch_step_narrow(const DeviceState& s, std::uint32_t waves, std::ui
 hipError_t launch_step(const DeviceState& state, std::uint32_t frameskip, std::uint32_t max_instr, int stats_mode,
                        hipStream_t stream) {
     DeviceState s = state;
-    if (stats_mode != 0 || budget_binds(max_instr) || s.n > kWaveMaxConsoles) s.choice = nullptr;
+    const std::uint32_t asked = asked_waves_per_group();
+    if (stats_mode != 0 || budget_binds(max_instr) || s.n > kWaveMaxConsoles || asked != 0) s.choice = nullptr;
     // One console per wave up to 32,768 consoles: there the wave kernel takes
     // 13.2 ms on a program that never idles and 4.75 on one that waits in
     // JMP *, this file's 17.3 and 5.98; at 40,960 16.7 and about 6 against
@@ -1543,7 +1545,7 @@ hipError_t launch_step(const DeviceState& state, std::uint32_t frameskip, std::u
                                                      : launch_step_wave(s, frameskip, stream);
         if (e != hipSuccess) return e;
     }
-    const std::uint32_t waves = waves_per_group();
+    const std::uint32_t waves = asked != 0 ? asked : 4u;
     const Geometry g = geometry(s.n, waves);
     if (g.full) return launch_step_full(s, frameskip, max_instr, stats_mode, stream);
     if (g.lds > kLdsLimit) return hipErrorInvalidConfiguration;

@@ -10,9 +10,11 @@ are compared with the oracle itself."""
 
 from __future__ import annotations
 
+import os
 import re
 import shutil
 import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -193,6 +195,21 @@ def test_ordinary_programs_stay_with_one_console_per_wave(n, chooses):
         b.set_actions(masks_for(9, n, k))
         b.step(stats_mode=1 if k == 2 else 0)
     assert b.step_choices() == ((4, 0) if chooses else (0, 0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value,chooses", [("8", False), ("16", False), ("5", True), ("", True)])
+def test_waves_per_group_asks_for_the_lane_kernel(value, chooses):
+    """NESLE_WAVES_PER_GROUP shapes the lane kernel's workgroups, so with a
+    value it takes (4, 8 or 16) that kernel runs; read once per process."""
+    say(f"[gpu] NESLE_WAVES_PER_GROUP={value!r}")
+    code = ("from nesle_amd import abi, synthrom; import numpy as np\n"
+            "b = abi.Batch(synthrom.make_rom(5).rom, 300, frameskip=1)\n"
+            "b.set_actions(np.zeros(300, np.uint8)); b.step(); b.step(); print(b.step_choices())")
+    out = subprocess.run([sys.executable, "-c", code], env={**os.environ, "NESLE_WAVES_PER_GROUP": value},
+                         cwd=build.ROOT, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.split("\n")[-2] == ("(2, 0)" if chooses else "(0, 0)"), out.stdout
 
 
 def vector_rom(irq: int, flow: list[int]) -> bytes:
