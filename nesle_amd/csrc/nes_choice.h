@@ -88,16 +88,33 @@ NESLE_BOTH_SIDES inline void choice_update(StepChoice& c) {
 }
 
 // Trips through the general path per frame from which on the lane kernel is
-// quicker on a batch of n consoles.  Per 1,024 consoles (one wave per SIMD) a
-// trip costs about 1,100 cycles of 2.4 GHz, and a step of four frames 0.42 ms,
-// at least 2.5 in all, against the lane kernel's 14 (up to 8,192 consoles) or
-// 17 ms: at 4,096 consoles 1,254 trips a frame, 8,192 580, 16,384 280,
-// 32,768 48.
-inline std::uint32_t general_limit(std::uint32_t n) {
-    const double waves = n > 1024 ? n / 1024.0 : 1.0;
-    const double lane_ms = n <= 8192 ? 14.0 : 17.0, wave_ms = 0.42 * waves > 2.5 ? 0.42 * waves : 2.5;
-    const double limit = (lane_ms - wave_ms) * 0.25e-3 * 2.4e9 * 0.8 / ((waves > 2.0 ? waves : 2.0) * 1100.0);
-    return limit > 0.0 ? static_cast<std::uint32_t>(limit) : 0u;
+// quicker on a batch of n consoles: `idle` of them, and `busy` more for a frame
+// that never waits in a jump to itself.  Both kernels skip those jumps, so a
+// program that waits for its NMI costs the lane kernel as little as its share
+// of a busy frame says, and fewer trips outweigh it.  In ms per step of four
+// frames, with w waves of one console per SIMD (1,024 consoles each), measured
+// on programs of 0 to 500 reads of $4015 a frame beside 60 to 2,600 other
+// instructions and a wait: the lane kernel 0.12 and, for a busy frame of 3.5
+// cycles an instruction, 15 up to 8,192 consoles or 18; one console per wave
+// 0.05 and 0.39 w, at least 2.4; a trip 1,660 cycles of 2.4 GHz per wave, of at
+// least 2.4 waves.  At 4,096 consoles 6 + 1,139 trips, 8,192 3 + 537, 16,384
+// 2 + 265, 32,768 1 + 62.
+struct GeneralLimit {
+    float idle, busy;
+};
+inline GeneralLimit general_limit(std::uint32_t n) {
+    const double w = n / 1024.0;
+    const double trip_ms = 4 * 1660.0 * (w > 2.4 ? w : 2.4) / 2.4e6;
+    const double lane_ms = n <= 8192 ? 15.0 : 18.0, wave_ms = 0.39 * w > 2.4 ? 0.39 * w : 2.4;
+    return {static_cast<float>((0.12 - 0.05) / trip_ms), static_cast<float>((lane_ms - wave_ms) / trip_ms)};
+}
+
+// Whether a console's step of `frames` frames, with `trips` trips and `jumps`
+// skipped jumps (9 dots each) of the frames' `dots`, is over it.
+NESLE_BOTH_SIDES inline bool over_limit(GeneralLimit l, std::uint32_t trips, std::uint32_t jumps, std::uint32_t frames,
+                                        std::uint32_t dots) {
+    const float n = static_cast<float>(frames), waits = 9.0f * static_cast<float>(jumps) / static_cast<float>(dots);
+    return static_cast<float>(trips) > l.idle * n + l.busy * (waits < n ? n - waits : 0.0f);
 }
 
 }  // namespace nesle

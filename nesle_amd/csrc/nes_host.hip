@@ -583,7 +583,9 @@ void open_batch(nesle_batch* b, const nesle_config* cfg) {
     s.clip = b->cfg.clip;
     s.time_penalty = b->cfg.time_penalty;
     b->closed_end = nesle::closed_end(b->rom.prg.data(), b->rom.prg.size());
-    s.general_limit = nesle::general_limit(s.n);
+    const nesle::GeneralLimit limit = nesle::general_limit(s.n);
+    s.general_idle = limit.idle;
+    s.general_busy = limit.busy;
     b->allocate();
     b->host_to_device(b->d_prg, b->rom.prg.data(), b->rom.prg.size(), "upload PRG ROM");
     if (!b->rom.chr.empty()) b->host_to_device(b->d_chr, b->rom.chr.data(), b->rom.chr.size(), "upload CHR ROM");

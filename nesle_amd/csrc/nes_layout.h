@@ -143,9 +143,9 @@ struct DeviceState {
     std::uint8_t* lat_ctrl;    // [n]
 
     // The choice between the step kernels (nes_choice.h), or null: the lane
-    // kernel.  And the trips through the general path per frame it turns on.
+    // kernel.  And the trips through the general path it turns on (GeneralLimit).
     StepChoice* choice;
-    std::uint32_t general_limit;
+    float general_idle, general_busy;
 };
 
 // Step-kernel census (stats mode 3): what the waves of one launch did, summed

@@ -24,7 +24,7 @@
 //
 // Statistics and binding instruction budgets stay with the lane kernel, as do
 // images whose flow can run past their end, and programs that take the general
-// path too often (nes_choice.h): an instruction there costs about 1,100
+// path too often (nes_choice.h): an instruction there costs 1,100 to 1,700
 // cycles of a SIMD, where a lane of the lane kernel shares 1,400 with 63
 // others.
 //
@@ -186,7 +186,7 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
         cpu.sp = uni(s.sp[env]); cpu.p = uni(s.p[env]);
         cpu.left = static_cast<std::int32_t>(uni(horizon0));
         __builtin_amdgcn_s_setprio(3);
-        std::uint32_t general = 0;   // trips through the general path
+        std::uint32_t general = 0, jumps = 0;   // trips through the general path, jumps of idle loops
         bool active = !(c.flags & kFault) && frameskip != 0;
         while (active) {
             const bool nmi = (c.flags & kNmiPending) != 0;
@@ -295,7 +295,11 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
                 cpu.a = regs & 0xFF; cpu.x = (regs >> 8) & 0xFF; cpu.y = (regs >> 16) & 0xFF; cpu.sp = regs >> 24;
                 // Idle loop (JMP to itself): the jumps until the next event in one go.
                 const std::int32_t gap = cpu.left - static_cast<std::int32_t>(dots);
-                if ((d14 & mc::kJmpAbs) && abs == pc0 && gap > 0) dots += 9u * static_cast<std::uint32_t>((gap + 8) / 9);
+                if ((d14 & mc::kJmpAbs) && abs == pc0 && gap > 0) {
+                    const std::uint32_t skipped = uni(static_cast<std::uint32_t>((gap + 8) / 9));
+                    dots += 9u * skipped;
+                    jumps += skipped;
+                }
                 if (d14 & mc::kIllegal) {
                     c.flags |= kFault;
                     active = false;
@@ -372,9 +376,11 @@ NESLE_WAVE_KERNEL(DeviceState s, std::uint32_t frameskip) {
         }
         flags = c.flags;
         frames = c.r32(reg::kFrames);
-        if (blockIdx.x < kGeneralSlots && wave == 0 && lane == 0 && frameskip != 0) {
+        // Whether the first consoles took the general path too often.
+        if (blockIdx.x < kGeneralSlots && wave == 0 && lane == 0) {
             KState* k = reload(c.s);
-            k->choice->over[blockIdx.x] = general / frameskip > k->general_limit ? 1u : 0u;
+            const GeneralLimit limit{k->general_idle, k->general_busy};
+            k->choice->over[blockIdx.x] = over_limit(limit, general, jumps, frameskip, kFrameDots) ? 1u : 0u;
         }
     }
     __syncthreads();

@@ -155,6 +155,35 @@ def test_polling_program_moves_to_the_lane_kernel(n):
     assert b.step_choices() == (2, 68)
 
 
+def waiting_rom(work: int, reads: int) -> bytes:
+    """An NMI handler of `work` turns of a loop and `reads` reads of $4015; the
+    main program waits in JMP *."""
+    turn = [0xB5, 0x10, 0x18, 0x75, 0x11, 0x95, 0x12, 0x0A, 0x2A, 0x65, 0x13, 0xCA]
+    read = [0xAD, 0x15, 0x40, 0x88]
+    nmi = [0xA2, work, *turn, 0xD0, 0x100 - len(turn) - 2, 0xA0, reads, *read, 0xD0, 0x100 - len(read) - 2, 0xE6, 0x20, 0x40]
+    reset = [0x78, 0xA2, 0xFF, 0x9A, 0xA9, 0x80, 0x8D, 0x00, 0x20, 0x4C, 0x09, 0x80]
+    return nrom_bytes(2, code={0x8000: reset, 0x9000: nmi}, reset=0x8000, nmi=0x9000, irq=0x9000)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("work,reads,stays", [(4, 5, True), (4, 100, False), (200, 100, True)])
+def test_waiting_programs_are_judged_by_their_share_of_a_frame(work, reads, stays):
+    """4,100 consoles (us per step of four frames, one console per wave against
+    lanes): 5 reads beside a long wait, 100 beside it (about 1,300 and 800),
+    100 beside 5,200 cycles of work (1,750 and 3,700)."""
+    n = 4100
+    say(f"[gpu] kernel choice: waiting program work={work} reads={reads} N={n}")
+    b = abi.Batch(waiting_rom(work, reads), n, frameskip=4)
+    b.set_actions(masks_for(8, n, 0))
+    b.set_lane_kernel(True)        # past power-on
+    for _ in range(2):
+        b.step()
+    b.set_lane_kernel(False)
+    for _ in range(2):
+        b.step()
+    assert b.step_choices() == ((2, 0) if stays else (1, 1))
+
+
 @pytest.mark.gpu
 def test_captured_steps_choose_when_they_run():
     """A step captured before any has run: the replays of its graph move to the
