@@ -77,37 +77,37 @@ HBM_PEAK_GBS = 8000.0
 VALU_PEAK_LANE_OPS = 256 * 4 * 16 * 2.4e9   # int32 lane-ops/s
 
 
-PROFILE = ROOT / "profiles" / "step_kernel_65536_fs4.md"
+# Largest batch the one-console-per-wave step kernels take.
+ONE_PER_WAVE_MAX = 32768
+PROFILE = ROOT / "profiles" / "step_kernel_65536_fs4.md"          # the lane kernel
+PROFILE_PER_WAVE = ROOT / "profiles" / "wave_kernel_fs4.md"       # one console per wave
 
 
 def profile_figure(key: str, num_envs: int) -> float | None:
     """A machine-readable figure (``<key> <envs> <value>``) of the committed
-    rocprofv3 summary, or None when the summary has none for this size."""
-    if not PROFILE.exists():
+    rocprofv3 summary of the kernel this size runs, or None when the summary
+    has none for it."""
+    path = PROFILE if num_envs > ONE_PER_WAVE_MAX else PROFILE_PER_WAVE
+    if not path.exists():
         return None
-    for line in PROFILE.read_text().splitlines():
+    for line in path.read_text().splitlines():
         parts = line.split()
         if len(parts) == 3 and parts[0] == key and parts[1] == str(num_envs):
             return float(parts[2])
     return None
 
 
-# Largest batch the one-console-per-wave step kernels take.
-ONE_PER_WAVE_MAX = 32768
-
-
 def size_figures(run: dict, num_envs: int) -> dict:
     """Throughput and roofline fractions of one batch size: NES frames/s,
     algorithmic and measured (rocprofv3, committed summary) HBM bytes per
-    kernel time against the 8 TB/s peak, and the VALU pipe's busy fraction."""
+    kernel time against the 8 TB/s peak, and how busy the instruction pipes are."""
     kernel_s = run["kernel_ms_per_launch"] / 1000.0
     algo = num_envs * B_STEP / kernel_s / 1e9
-    # The summary's counters are the lane kernel's.
-    counted = num_envs > ONE_PER_WAVE_MAX
-    traffic = profile_figure("traffic_bytes_per_launch", num_envs) if counted else None
+    traffic = profile_figure("traffic_bytes_per_launch", num_envs)
     measured = traffic / kernel_s / 1e9 if traffic else None
-    lane_ops = profile_figure("valu_lane_ops_per_launch", num_envs) if counted else None
+    lane_ops = profile_figure("valu_lane_ops_per_launch", num_envs)
     lanes = consoles_per_wave(num_envs)
+    in_lanes = num_envs > ONE_PER_WAVE_MAX
     return {
         "num_envs": num_envs,
         "env_steps_per_s": run["env_steps_per_s"],
@@ -118,13 +118,16 @@ def size_figures(run: dict, num_envs: int) -> dict:
         "hbm_algorithmic_frac": algo / HBM_PEAK_GBS,
         "hbm_measured_gbs": measured,
         "hbm_measured_frac": measured / HBM_PEAK_GBS if measured else None,
-        "valu_busy_frac": profile_figure("valu_busy", num_envs) if counted else None,
+        "valu_busy_frac": profile_figure("valu_busy", num_envs),
+        "salu_busy_frac": profile_figure("salu_busy", num_envs),
         "valu_lane_ops_frac": lane_ops / kernel_s / VALU_PEAK_LANE_OPS if lane_ops else None,
         "consoles_per_wave": lanes,
-        # Lanes without a console run the datapath on a dummy block: only
-        # lanes/64 of the VALU lane-ops serve a console.
-        "useful_lane_frac": lanes / 64,
-        "useful_valu_lane_ops_frac": lane_ops / kernel_s / VALU_PEAK_LANE_OPS * lanes / 64 if lane_ops else None,
+        # The lane kernel's lanes without a console run the datapath on a dummy
+        # block: only lanes/64 of the VALU lane-ops serve a console.  One
+        # console per wave runs on the scalar unit, with one lane active.
+        "useful_lane_frac": lanes / 64 if in_lanes else None,
+        "useful_valu_lane_ops_frac": lane_ops / kernel_s / VALU_PEAK_LANE_OPS * lanes / 64
+        if lane_ops and in_lanes else None,
     }
 
 
