@@ -246,13 +246,14 @@ struct nesle_batch {
     std::uint64_t timed_launches = 0;
     // The choice between the step kernels (nes_choice.h).
     bool closed_end = false, lanes_only = false;
-    // Pinned host memory that kernels read and write: the actions of a step on
-    // their way in, small views on their way out.  A copy between pageable
-    // memory and the device waits for the stream, and costs 25-45 us of its
-    // own; through here the actions wait for nothing and the views of a call
+    // Pinned host memory that kernels read and write: a step's actions and a
+    // reset's mask on their way in, small views on their way out.  A copy between
+    // pageable memory and the device waits for the stream, and costs 25-45 us of
+    // its own; through here the actions wait for nothing and the views of a call
     // for one kernel (steps of the vector environment: 1 console with RGB 784 ->
-    // 725 us, 64 with RAM 797 -> 760).  Copies
-    // above kStageMax go straight, as their bytes outweigh the wait.
+    // 725 us, 64 with RAM 797 -> 760).  Views that do not fit beside the ones
+    // before them go straight, as their bytes outweigh the wait; the small ones
+    // of the call do not (6 consoles with RGB, frame-skip 1: 315 -> 296 us).
     static constexpr std::size_t kStageMax = std::size_t{1} << 20;
     std::mutex stage_mutex;             // one copy at a time
     std::uint8_t* stage_in = nullptr;   // n bytes, and behind them
@@ -391,10 +392,10 @@ struct nesle_batch {
         return status == hipStreamCaptureStatusNone;
     }
 
-    // The actions of a step, one byte per console, from host memory.
-    void upload_actions(std::uint8_t* dst, const std::uint8_t* src) {
+    // One byte per console from host memory: a step's actions, a reset's mask.
+    void upload(std::uint8_t* dst, const std::uint8_t* src, const char* what) {
         if (!staged()) {
-            host_to_device(dst, src, n(), "copy actions");
+            host_to_device(dst, src, n(), what);
             return;
         }
         std::lock_guard<std::mutex> lock(stage_mutex);
@@ -405,7 +406,7 @@ struct nesle_batch {
         c.src[0] = stage_in;
         c.dst[0] = dst;
         c.bytes[0] = n();
-        hip_check(nesle::launch_stage_copy(c, 1, stream), "copy actions");
+        hip_check(nesle::launch_stage_copy(c, 1, stream), what);
     }
 
     struct HostCopy {
@@ -415,29 +416,30 @@ struct nesle_batch {
     };
     // Device buffers to host memory, with one wait.
     void download(const HostCopy* copies, std::uint32_t count) {
-        std::size_t total = 0;
-        for (std::uint32_t i = 0; i < count; ++i) total += align_up(copies[i].bytes, 256);
-        if (count > nesle::kStageCopies || total > stage_bytes || !staged()) {
-            for (std::uint32_t i = 0; i < count; ++i)
-                hip_check(hipMemcpyAsync(copies[i].dst, copies[i].src, copies[i].bytes, hipMemcpyDeviceToHost, stream),
-                          "copy view to host");
-            sync();
-            return;
-        }
-        std::lock_guard<std::mutex> lock(stage_mutex);
+        std::unique_lock<std::mutex> lock(stage_mutex);
+        const std::size_t room = staged() ? stage_bytes : 0;
         nesle::StageCopy c{};
+        void* to[nesle::kStageCopies];
+        std::uint32_t through = 0;   // views that go through pinned memory
         std::size_t at = 0;
+        std::vector<HostCopy> straight;
         for (std::uint32_t i = 0; i < count; ++i) {
-            c.src[i] = static_cast<const std::uint8_t*>(copies[i].src);
-            c.dst[i] = stage_out + at;
-            c.bytes[i] = static_cast<std::uint32_t>(copies[i].bytes);
+            if (through == nesle::kStageCopies || at + copies[i].bytes > room) {
+                straight.push_back(copies[i]);
+                continue;
+            }
+            c.src[through] = static_cast<const std::uint8_t*>(copies[i].src);
+            c.dst[through] = stage_out + at;
+            c.bytes[through] = static_cast<std::uint32_t>(copies[i].bytes);
+            to[through++] = copies[i].dst;
             at += align_up(copies[i].bytes, 256);
         }
-        hip_check(nesle::launch_stage_copy(c, count, stream), "copy view to host");
+        if (through != 0) hip_check(nesle::launch_stage_copy(c, through, stream), "copy view to host");
+        for (const auto& s : straight)
+            hip_check(hipMemcpyAsync(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost, stream), "copy view to host");
         sync();
         stage_in_busy = false;
-        for (std::uint32_t i = 0; i < count; ++i)
-            std::memcpy(copies[i].dst, c.dst[i], copies[i].bytes);
+        for (std::uint32_t i = 0; i < through; ++i) std::memcpy(to[i], c.dst[i], c.bytes[i]);
     }
 
     std::uint8_t* frame_buffer(int output) {
@@ -718,7 +720,7 @@ int nesle_reset_envs(nesle_batch* b, const std::uint8_t* mask, int mask_on_devic
         b->activate();
         const std::uint8_t* dmask = mask;
         if (!mask_on_device) {
-            b->host_to_device(b->d_mask, mask, b->n(), "copy reset mask");
+            b->upload(b->d_mask, mask, "copy reset mask");
             dmask = b->d_mask;
         }
         if (b->synthetic)
@@ -740,7 +742,7 @@ int nesle_set_actions(nesle_batch* b, const void* actions, int dtype, int on_dev
             if (on_device) {
                 hip_check(hipMemcpyAsync(dst, actions, n, hipMemcpyDeviceToDevice, b->stream), "copy actions");
             } else {
-                b->upload_actions(dst, static_cast<const std::uint8_t*>(actions));
+                b->upload(dst, static_cast<const std::uint8_t*>(actions), "copy actions");
             }
         } else if (dtype == NESLE_DTYPE_I64) {
             if (on_device) {
@@ -750,7 +752,7 @@ int nesle_set_actions(nesle_batch* b, const void* actions, int dtype, int on_dev
                 std::vector<std::uint8_t> tmp(n);
                 const auto* src = static_cast<const long long*>(actions);
                 for (std::size_t i = 0; i < n; ++i) tmp[i] = static_cast<std::uint8_t>(src[i] & 0xFF);
-                b->upload_actions(dst, tmp.data());
+                b->upload(dst, tmp.data(), "copy actions");
             }
         } else {
             throw InvalidArgument("actions must be uint8 masks or int64 values already encoded as masks");

@@ -191,9 +191,10 @@ def test_ram_device_matches_oracle_after_steps():
         assert np.array_equal(ram[e], o.save()[O.OFF["ram"]:O.OFF["ram"] + 2048])
 
 
-# Actions in and views out through pinned memory up to 1 MiB, straight above:
-# a batch of each, on its own stream, its pads overwritten right after the
-# call that took them.
+# Actions and reset masks in and views out through pinned memory up to 1 MiB,
+# straight above (six frames: the rewards and dones beside them still through
+# it): a batch of each, on its own stream, its pads and mask overwritten right
+# after the call that took them.
 @pytest.mark.parametrize("num_envs,frames", [(1, True), (5, True), (6, True), (63, False), (511, False), (513, False)])
 def test_host_step_matches_device_step(num_envs, frames):
     import torch
@@ -215,3 +216,10 @@ def test_host_step_matches_device_step(num_envs, frames):
         assert np.array_equal(got["rewards"], torch.from_dlpack(b.rewards_device()).cpu().numpy())
         assert np.array_equal(got["dones"], torch.from_dlpack(b.last_done_device()).cpu().numpy())
         assert np.array_equal(got["obs"], b.render() if frames else b.ram())
+    mask = (np.arange(num_envs) % 3 == 0).astype(np.uint8)
+    want = torch.from_numpy(mask.copy()).cuda()
+    a.reset_envs(mask)
+    mask[:] = 1
+    b.reset_envs_device(want)
+    b.synchronize()
+    assert np.array_equal(a.ram(), torch.from_dlpack(b.ram_device()).cpu().numpy())
